@@ -1,15 +1,15 @@
-// Dense fp32 MFMA GEMM (om_gemm), the Linear layer forward/backward built on it, and the split-K reduction.
+// Dense products (om_gemm), the Linear layer forward/backward built on them, and the split-K reduction.
 //
-// Tile selection is a function of the shape and the CU count only. Well-aligned operands (every pointer 16-byte
-// aligned, leading dimensions multiples of 4) run the BK = 32 "fast set" of tiles; anything else runs 64 x 64 tiles
-// with element-guarded loads. The chooser prefers tilings whose workgroup count fills whole rounds of the 256 CUs
-// (128 x 192 for 4096 x 1536 gives exactly 256 tiles, 64 x 96 for 4096 x 384 likewise), because a last round that
-// is half empty costs as much as a full one.
+// A product runs the split-operand kernel (om_gemm_s.hpp) on a tile and a K split that depend on the shape and the CU
+// count only (choose_s); short sums over few whole tiles run the tile-exact fp32 kernels (om_gemm_x.hpp, short_tile);
+// what neither takes (both operands transposed, fewer than four columns, sums of fewer than 16 terms, leading dimensions
+// past 32-bit byte offsets) the guarded fp32 kernel k_gemm.
 #include <cstdlib>
 #include <cstring>
 #include <utility>
 
 #include "om_gemm.hpp"
+#include "om_gemm_s.hpp"
 #include "om_gemm_x.hpp"
 
 namespace omg {
@@ -181,15 +181,6 @@ static void launch_t(const Params &p, int batch, hipStream_t st) {
     hipLaunchKernelGGL((k_gemm<BM, BN, BKT, TA, TB, VEC>), dim3((unsigned)total), dim3(NT), 0, st, p);
 }
 
-// Fast set: aligned operands, BK = 32, the three layouts the training path uses (NN, NT, TN).
-template <int BM, int BN>
-static bool launch_fast(const Params &p, int batch, bool ta, bool tb, hipStream_t st) {
-    if (!ta && !tb) launch_t<BM, BN, 32, false, false, true>(p, batch, st);
-    else if (!ta && tb) launch_t<BM, BN, 32, false, true, true>(p, batch, st);
-    else if (ta && !tb) launch_t<BM, BN, 32, true, false, true>(p, batch, st);
-    else return false;
-    return true;
-}
 // General set: any layout and alignment, BK = 16.
 template <int BM, int BN>
 static void launch_general(const Params &p, int batch, bool ta, bool tb, bool vec, hipStream_t st) {
@@ -206,308 +197,83 @@ static void launch_general(const Params &p, int batch, bool ta, bool tb, bool ve
 #undef OMG_CASE
 }
 
-// The epilogues only some tile instances carry: GELU and its backward terms. EPI_RELU, like the bias and the
-// residual, is applied by every instance. An instance's epilogue family GK is 0 (none of them), 1 (the reference's
-// polynomials: EPI_GELU, EPI_GELU_GRAD, EPI_GELU_SLOPE) or 2 (the same with erf and exp of stated error:
-// EPI_GELU_F, EPI_GELU_GRAD_F, EPI_GELU_SLOPE_F); both families also carry EPI_MUL_AUX (no transcendental).
-static bool gelu_epi(int epi) { return epi != EPI_NONE && epi != EPI_RELU; }
-// 1 or 2: the family the epilogue needs; 3: either (EPI_MUL_AUX); 0: none.
-static int epi_family(int epi) {
-    if (epi == EPI_GELU || epi == EPI_GELU_GRAD || epi == EPI_GELU_SLOPE) return 1;
-    if (epi == EPI_GELU_F || epi == EPI_GELU_GRAD_F || epi == EPI_GELU_SLOPE_F) return 2;
-    return epi == EPI_MUL_AUX ? 3 : 0;
-}
-// The family an instance set GM (bit 0: family 1 instantiated, bit 1: family 2) runs epilogue `epi` with, or -1.
-static int pick_family(int GM, int epi) {
-    const int f = epi_family(epi);
-    if (f == 0) return 0;
-    if (f == 3) return (GM & 2) ? 2 : (GM & 1) ? 1 : -1;
-    return (GM & f) ? f : -1;
-}
-
-// In a tuning build (om::tuning_env), OM_GEMM_DMA=0 keeps NT products on k_gemm_x's register-staged loads and
-// OM_GEMM_DMA=2 puts every NT product with 32-deep chunks (plain or fast GELU) on k_gemm_xd, whose chunks load
-// straight into LDS, however many rounds its tiles take (for comparisons); otherwise launch_x's rule decides.
-static bool dma_disabled() {
-    static const char *s = om::tuning_env("OM_GEMM_DMA");
-    return s && s[0] == '0';
-}
-static bool dma_forced() {
-    static const char *s = om::tuning_env("OM_GEMM_DMA");
-    return s && s[0] == '2';
-}
-
-// Launches kernel K with the epilogue family gk, instantiating only the families GM holds.
-#define OMG_L(K, NTH, TA_, TB_)                                                                                  \
-    do {                                                                                                         \
-        if constexpr ((GM & 1) != 0)                                                                             \
-            if (gk == 1) {                                                                                       \
-                hipLaunchKernelGGL((gx::K<BM, BN, BKT, TA_, TB_, 1>), dim3(total), dim3(NTH), 0, st, p);         \
-                break;                                                                                           \
-            }                                                                                                    \
-        if constexpr ((GM & 2) != 0)                                                                             \
-            if (gk == 2) {                                                                                       \
-                hipLaunchKernelGGL((gx::K<BM, BN, BKT, TA_, TB_, 2>), dim3(total), dim3(NTH), 0, st, p);         \
-                break;                                                                                           \
-            }                                                                                                    \
-        hipLaunchKernelGGL((gx::K<BM, BN, BKT, TA_, TB_, 0>), dim3(total), dim3(NTH), 0, st, p);                 \
-    } while (0);
-
-// Tile-exact set (om_gemm_x.hpp): NN, NT, TN; GELU epilogue variants (NN / NT only) of the families GM holds.
-template <int BM, int BN, int BKT, int GM>
-static bool launch_x(const Params &p, int batch, bool ta, bool tb, hipStream_t st, int cus, int dma) {
-    const unsigned total = (unsigned)((int64_t)(p.m / BM) * (p.n / BN) * batch * p.splits);
-    const int gk = pick_family(GM, p.epi);
-    if (gk < 0 || (gk > 0 && ta)) return false;
-    if (!ta && !tb) {
-        OMG_L(k_gemm_x, NT, false, false)
-    } else if (!ta && tb) {
-        // Both operands K-contiguous: chunks load straight into LDS, when the grid fits in one round of the CUs at
-        // the occupancy the three LDS stages allow (C3: the 256-tile products gain 7-8 %, the 768-tile q|k|v
-        // projection would lose 14 % to a second round), or when the tuned table asks for it (dma): the FFN's first
-        // products and C5's q|k|v projection, several rounds, plain or with the fast GELU pair (3-7 % faster). Not
-        // for the reference's polynomials, whose element-wise tail hides better behind the register-staged kernel's
-        // higher occupancy (75 against 81 us for the C3 FFN product).
-        if constexpr (BKT == 32) {
-            constexpr int lds = 4 * (64 + 3 * (BM + BN) * BKT);
-            const unsigned per_cu = (160u << 10) / lds;
-            const bool want = (gk == 0 && total <= per_cu * (unsigned)cus) || ((dma || dma_forced()) && gk != 1);
-            if (want && !dma_disabled()) {
-                if constexpr ((GM & 2) != 0)
-                    if (gk == 2) {
-                        hipLaunchKernelGGL((gx::k_gemm_xd<BM, BN, BKT, 2>), dim3(total), dim3(NT), 0, st, p);
-                        return true;
-                    }
-                if (gk == 0) {
-                    hipLaunchKernelGGL((gx::k_gemm_xd<BM, BN, BKT, 0>), dim3(total), dim3(NT), 0, st, p);
-                    return true;
-                }
-            }
-        }
-        OMG_L(k_gemm_x, NT, false, true)
-    } else if (ta && !tb) {
-        hipLaunchKernelGGL((gx::k_gemm_x<BM, BN, BKT, true, false, 0>), dim3(total), dim3(NT), 0, st, p);
-    } else {
-        return false;
-    }
-    return true;
-}
-// Eight-wavefront variant (om_gemm_x.hpp, k_gemm_x2).
-template <int BM, int BN, int BKT, int GM>
-static bool launch_x2(const Params &p, int batch, bool ta, bool tb, hipStream_t st) {
-    const unsigned total = (unsigned)((int64_t)(p.m / BM) * (p.n / BN) * batch * p.splits);
-    const int gk = pick_family(GM, p.epi);
-    if (gk < 0 || (gk > 0 && ta)) return false;
-    if (!ta && !tb) {
-        OMG_L(k_gemm_x2, 2 * NT, false, false)
-    } else if (!ta && tb) {
-        OMG_L(k_gemm_x2, 2 * NT, false, true)
-    } else if (ta && !tb) {
-        hipLaunchKernelGGL((gx::k_gemm_x2<BM, BN, BKT, true, false, 0>), dim3(total), dim3(2 * NT), 0, st, p);
-    } else {
-        return false;
-    }
-    return true;
-}
-#undef OMG_L
-
-struct XTile {
-    int bm, bn, bkt;
-    int dma = 0;  // Choice::dma
-};
-// Launches tile t; false when t (or its variant for the product's epilogue) is not instantiated.
-static bool dispatch_x(const XTile &t, const Params &p, int batch, bool ta, bool tb, hipStream_t st, int cus) {
-    // bkt 33 / 65 select the eight-wavefront variant of the 32 / 64 chunk. The last template argument lists the
-    // GELU epilogue families the tile instantiates (bit 0: the reference's polynomials, bit 1: the fast pair).
-    if (t.bkt == 33 && t.bm == 64 && t.bn == 96) return launch_x2<64, 96, 32, 3>(p, batch, ta, tb, st);
-    if (t.bkt == 33 && t.bm == 64 && t.bn == 64) return launch_x2<64, 64, 32, 1>(p, batch, ta, tb, st);
-    if (t.bkt == 65 && t.bm == 64 && t.bn == 96) return launch_x2<64, 96, 64, 0>(p, batch, ta, tb, st);
-    if (t.bkt == 33 && t.bm == 128 && t.bn == 128) return launch_x2<128, 128, 32, 2>(p, batch, ta, tb, st);
-    if (t.bkt == 33 && t.bm == 128 && t.bn == 96) return launch_x2<128, 96, 32, 3>(p, batch, ta, tb, st);
-#define OMG_X(BM, BN, BKT, GM) \
-    if (t.bm == BM && t.bn == BN && t.bkt == BKT) return launch_x<BM, BN, BKT, GM>(p, batch, ta, tb, st, cus, t.dma);
-    OMG_X(64, 64, 32, 3)
-    OMG_X(64, 96, 32, 3)
-    OMG_X(96, 64, 32, 0)
-    OMG_X(64, 128, 32, 2)
-    OMG_X(128, 64, 32, 2)
-    OMG_X(128, 96, 32, 3)
-    OMG_X(128, 128, 32, 2)
-    OMG_X(64, 64, 64, 1)
-    OMG_X(64, 96, 64, 0)
-    OMG_X(128, 128, 64, 0)
-#undef OMG_X
-    return false;
-}
-
-// Whether tile t covers the product exactly (full tiles, whole chunks per split, 32-bit in-tile offsets).
-static bool x_fits(const XTile &t, const Params &p, int splits, int k_split) {
-    const int ck = t.bkt & ~1;  // chunk depth (an odd bkt selects the eight-wavefront variant)
-    if (p.m % t.bm || p.n % t.bn || p.k % ck || k_split % ck) return false;
-    if (splits > 1 && (int64_t)(splits - 1) * k_split >= p.k) return false;
-    const int64_t ld = p.lda > p.ldb ? p.lda : p.ldb;
-    const int rows = t.bm > t.bn ? t.bm : t.bn;
-    return ld * (rows > ck ? rows : ck) < (int64_t)1 << 31;
-}
-
 namespace {
-// Tuned choices for the products of the training path's configurations (MI355X, random operands, one sweep of
-// the tile-exact kernels over tiles x chunk depths x split counts; C5's 768-wide rows re-swept with the 128 x 96
-// tile, which makes 4096 x 768 exactly one tile per CU: 8 % faster for the FFN's second product and the attention
-// output, 2-3 % for the q|k|v projection and two input gradients): exact shape -> tile and split count.
-struct Tuned {
-    int m, n, k;
-    bool ta, tb;
-    int bm, bn, bkt, splits;
-    int dma = 0;  // Choice::dma
-};
-const Tuned kTuned[] = {
-    // Linear forward y = x W^T (NT)
-    {4096, 384, 384, false, true, 64, 96, 32, 1},     {4096, 1536, 384, false, true, 64, 96, 32, 1, 1},
-    {4096, 384, 1536, false, true, 64, 96, 32, 1},    {4096, 1152, 384, false, true, 64, 96, 32, 1},
-    {4096, 768, 768, false, true, 128, 96, 32, 1},    {4096, 3072, 768, false, true, 128, 128, 32, 1, 1},
-    {4096, 768, 3072, false, true, 128, 96, 32, 1},   {4096, 2304, 768, false, true, 64, 96, 32, 1, 1},
-    // input gradient dx = g W (NN); bkt 33 = the eight-wavefront kernel with 32-deep chunks
-    {4096, 384, 384, false, false, 64, 96, 33, 1},    {4096, 384, 1536, false, false, 64, 96, 33, 1},
-    {4096, 1536, 384, false, false, 64, 64, 33, 1},   {4096, 384, 1152, false, false, 64, 96, 33, 1},
-    {4096, 768, 768, false, false, 64, 64, 32, 1},    {4096, 768, 3072, false, false, 128, 96, 33, 1},
-    {4096, 3072, 768, false, false, 128, 128, 33, 1}, {4096, 768, 2304, false, false, 128, 96, 33, 1},
-    // weight gradient dW = g^T x (TN), K = tokens
-    {384, 384, 4096, true, false, 64, 96, 33, 8},     {1536, 384, 4096, true, false, 64, 96, 32, 8},
-    {384, 1536, 4096, true, false, 64, 96, 32, 8},    {1152, 384, 4096, true, false, 64, 64, 32, 4},
-    {768, 768, 4096, true, false, 64, 96, 32, 8},     {3072, 768, 4096, true, false, 64, 96, 32, 2},
-    {768, 3072, 4096, true, false, 64, 96, 32, 2},    {2304, 768, 4096, true, false, 64, 96, 32, 2},
-};
-// The same for products with a GELU epilogue (GELU and its slope in the forward, the slope product in the input
-// gradient), whose element-wise tail shifts the best tile: the reference's polynomials (family 1) and the slope
-// product beside them ...
-const Tuned kTunedEpi[] = {
-    {4096, 1536, 384, false, true, 64, 64, 32, 1},
-    {4096, 1536, 384, false, false, 64, 96, 33, 1},
-};
-// ... and the fast pair (family 2) with its slope product, whose shorter tail lets the wide tiles of the plain
-// products through. The forward products run on the direct-to-LDS kernel; their tiles were picked by the step time
-// (C3 0.5304 ms at 64 x 64 against 0.5310 at 64 x 96 and 0.5333 for the register-staged 128 x 96; C5 7.166 ms at
-// 64 x 96 against 7.199 at 128 x 128 and 7.185 register-staged), which ranks them differently from the products
-// timed alone on warm operands.
-const Tuned kTunedGeluFast[] = {
-    {4096, 1536, 384, false, true, 64, 64, 32, 1, 1}, {4096, 3072, 768, false, true, 64, 96, 32, 1, 1},
-    {4096, 1536, 384, false, false, 64, 96, 33, 1},   {4096, 3072, 768, false, false, 64, 64, 32, 1},
-};
-
 // K length of one split: k / splits rounded up to whole chunks.
-int split_len(int k, int splits, int bkt) { return ((k + splits - 1) / splits + bkt - 1) / bkt * bkt; }
+int split_len(int k, int splits, int chunk) { return ((k + splits - 1) / splits + chunk - 1) / chunk * chunk; }
 
-Choice with_splits(int bm, int bn, int bkt, int k, int splits) {
-    Choice c{bm, bn, 1, k, bkt};
-    if (splits > 1) {
-        c.k_split = split_len(k, splits, bkt & ~1);
-        c.splits = (k + c.k_split - 1) / c.k_split;
-        if (c.splits <= 1) c.k_split = k;
-    }
-    return c;
-}
-
-// Tuning builds (om::tuning_env): OM_GEMM_X="bm,bn,bkt[,splits]" forces a tile-exact configuration where it fits (read
-// at every call, so one process can compare configurations).
-bool env_override(Choice &c, int k) {
-    const char *s = om::tuning_env("OM_GEMM_X");
-    if (!s || !*s || !strcmp(s, "off")) return false;
-    int bm = 0, bn = 0, bk = 32, sp = 1;
-    if (sscanf(s, "%d,%d,%d,%d", &bm, &bn, &bk, &sp) < 3) return false;
-    c = with_splits(bm, bn, bk, k, sp);
-    return true;
-}
-// Tile order of the grouped weight gradients: bands of 8 tile rows walked column by column when the group runs
-// unsplit (C5's layers: 1728 tiles, 517 -> ~490 us per launch, the step 7.37 -> 7.26 ms), row-major when it splits K
-// (C3's four products: banding cut the fetch but slowed the step). Tuning builds read OM_GROUP_BAND (0: row-major).
-int group_band(int splits) {
-    static const int b = [] {
-        const char *s = om::tuning_env("OM_GROUP_BAND");
-        return s && *s ? atoi(s) : -1;
-    }();
-    return b >= 0 ? b : (splits == 1 ? 8 : 0);
-}
-bool x_disabled() {
-    const char *s = om::tuning_env("OM_GEMM_X");
-    return s && !strcmp(s, "off");
-}
-// Tuning builds: OM_GEMM_T="m,n,k,ta,tb,family:bm,bn,bkt,splits,dma;..." replaces the tuned choice of the products of
-// exactly that shape and epilogue family (for step-level comparisons of one product's tile).
-struct ShapeOverride {
-    int m, n, k, ta, tb, fam, bm, bn, bkt, splits, dma;
+// The split-operand kernel's tiles (OMG_S_CONFIGS) and what the chooser knows of them, measured on MI355X with random
+// operands: `cost` is the CU time of one 32 x 32 x 32 block of the tile in units of 0.08 us (the wide tiles' rate: 256 x
+// 96 at 2.2 us and 128 x 96 at 0.95 us per 32-k step), `per_cu` the workgroups a CU holds. Splitting B once for more
+// rows, or A for more columns, is what makes the wide tiles cheaper; the k-group tiles pay for their extra splits and the
+// sum over groups, and earn it where wide tiles would leave CUs idle (4096 x 384 x 1536: 64 x 96 with four groups 35.5
+// us, 128 x 96 51.7 us; 4096 x 1536 x 384: 256 x 96 32.6 us, 64 x 96 49 us).
+struct SConfig {
+    int id, bm, bn, kg, waves;
+    double cost, alone;  // the cost beside other workgroups on the CU, and of one that has the CU to itself
+    int per_cu;
 };
-const std::vector<ShapeOverride> &shape_overrides() {
-    static const std::vector<ShapeOverride> v = [] {
-        std::vector<ShapeOverride> out;
-        const char *s = om::tuning_env("OM_GEMM_T");
-        while (s && *s) {
-            ShapeOverride o{};
-            if (sscanf(s, "%d,%d,%d,%d,%d,%d:%d,%d,%d,%d,%d", &o.m, &o.n, &o.k, &o.ta, &o.tb, &o.fam, &o.bm, &o.bn,
-                       &o.bkt, &o.splits, &o.dma) == 11)
-                out.push_back(o);
-            s = strchr(s, ';');
-            if (s) s++;
-        }
-        return out;
-    }();
-    return v;
-}
-}  // namespace
+const SConfig kS[] = {
+    {0, 256, 128, 1, 8, 1.02, 1.02, 1}, {1, 256, 96, 1, 8, 1.0, 1.0, 1},  {2, 128, 128, 1, 4, 1.02, 1.05, 2},
+    {3, 128, 96, 1, 4, 1.03, 1.12, 2},  {4, 128, 64, 1, 4, 1.15, 1.6, 2}, {5, 64, 96, 4, 8, 1.3, 1.3, 1},
+    {6, 64, 64, 4, 8, 1.35, 1.35, 1},   {7, 64, 64, 2, 4, 1.3, 1.8, 2},
+};
+// Split counts the reduce is built for.
+const int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 12, 16};
 
-// Aligned operands: the tuned table for the training path's products, else the rule it was distilled into
-// (MI355X measurements, random operands):
-//   - long-K products with few 64 x 64 tiles (weight gradients, K = tokens) split K into a power-of-two number of
-//     slices of at least 256 k, with tiles x splits near three workgroups per CU (64 x 96 tiles when N allows);
-//   - otherwise 64 x 96 when N is a multiple of 96 and its tiles fit in one round of the CUs (4096 x 384 becomes
-//     exactly 256 tiles: one per CU), else 64 x 64 (occupancy 4, best once there are several tiles per CU).
-Choice choose_fast(int m, int n, int k, int batch, bool ta, bool tb, int cus, int family) {
-    Choice best{64, 64, 1, k, 32};
-    if (env_override(best, k)) return best;
-    for (const ShapeOverride &o : shape_overrides())
-        if (o.m == m && o.n == n && o.k == k && o.ta == (int)ta && o.tb == (int)tb && o.fam == family && batch == 1) {
-            Choice c = with_splits(o.bm, o.bn, o.bkt, k, o.splits);
-            c.dma = o.dma;
-            return c;
+// Estimated time (units of 0.08 us) of products of `tiles` workgroups in all, each `steps` 32-k steps long: every CU's
+// share of tiles, a fixed cost of each round of workgroups (first loads, epilogue; about 3 us), and with a split the
+// reduce (a launch, then the partial sums it reads at about 5 TB/s).
+double s_time(const SConfig &c, int64_t tiles, int steps, int cus) {
+    const int64_t share = (tiles + cus - 1) / cus, rounds = (tiles + (int64_t)cus * c.per_cu - 1) / ((int64_t)cus * c.per_cu);
+    const int blocks = c.bm * c.bn / 1024, st = (steps + c.kg - 1) / c.kg * c.kg;
+    return (double)share * blocks * (st * (share > 1 ? c.cost : c.alone) + 1.5) + 38.0 * (double)rounds;
+}
+double reduce_time(int splits, double outputs) {
+    return splits > 1 ? 25.0 + (splits + 1.0) * outputs * 4.0 / 5.0e6 / 0.08 : 0.0;
+}
+struct SChoice {
+    const SConfig *c;
+    int splits, k_split;
+    bool exact;  // whole tiles and the same whole number of 32-k steps for every k group
+};
+// Tile and split of `count` products (m_i x n_i) over a common k (one product, or a weight-gradient group), each `batch`
+// times: the least s_time + reduce_time, the first on a tie.
+SChoice choose_s(int count, const int *m, const int *n, int k, int batch, int cus, bool may_split) {
+    SChoice best{&kS[0], 1, k, false};
+    double best_t = 1e300, outputs = 0.0;
+    for (int i = 0; i < count; i++) outputs += (double)m[i] * n[i];
+    for (const SConfig &c : kS) {
+        int64_t tiles = 0;
+        bool whole = true;
+        for (int i = 0; i < count; i++) {
+            tiles += (int64_t)((m[i] + c.bm - 1) / c.bm) * ((n[i] + c.bn - 1) / c.bn) * batch;
+            whole = whole && m[i] % c.bm == 0 && n[i] % c.bn == 0;
         }
-    if (batch == 1 && family == 2)
-        for (const Tuned &t : kTunedGeluFast)
-            if (t.m == m && t.n == n && t.k == k && t.ta == ta && t.tb == tb) {
-                Choice c = with_splits(t.bm, t.bn, t.bkt, k, t.splits);
-                c.dma = t.dma;
-                return c;
+        for (const int sp : kSplits) {
+            if (sp > 1 && (!may_split || batch > 1 || k / sp < 32 * c.kg)) break;
+            const int len = sp > 1 ? split_len(k, sp, 32 * c.kg) : k;
+            if (sp > 1 && (int64_t)(sp - 1) * len >= k) continue;
+            const bool exact = whole && k % (32 * c.kg) == 0;
+            const double t = (s_time(c, tiles * sp, (len + 31) / 32, cus) * (exact ? 1.0 : 1.08)) + reduce_time(sp, outputs);
+            if (t < best_t) {
+                best_t = t;
+                best = SChoice{&c, sp, len, exact};
             }
-    if (batch == 1 && family == 1)
-        for (const Tuned &t : kTunedEpi)
-            if (t.m == m && t.n == n && t.k == k && t.ta == ta && t.tb == tb)
-                return with_splits(t.bm, t.bn, t.bkt, k, t.splits);
-    if (batch == 1)
-        for (const Tuned &t : kTuned)
-            if (t.m == m && t.n == n && t.k == k && t.ta == ta && t.tb == tb) {
-                Choice c = with_splits(t.bm, t.bn, t.bkt, k, t.splits);
-                c.dma = t.dma;
-                return c;
-            }
-    const bool n96 = n % 96 == 0 && m >= 64;
-    int64_t tiles = (int64_t)((m + 63) / 64) * (n96 ? n / 96 : (n + 63) / 64) * batch;
-    // A handful of tiles over a long-enough K (an MLP's first layer: 4 tiles over K = 784) leaves most CUs idle, and
-    // each workgroup's chunks then follow one another at memory latency: split K into slices of at least 64 k until
-    // there are about as many workgroups as CUs / 2.
-    if (batch == 1 && 8 * tiles <= cus && k >= 256) {
-        int s = 1;
-        while (s < 16 && k / (2 * s) >= 64 && tiles * 2 * s <= cus / 2) s *= 2;
-        if (s > 1) return with_splits(64, 64, 32, k, s);
+        }
     }
-    if (batch == 1 && tiles < 2 * cus && k >= 1024) {
-        double want = 3.0 * cus / (double)tiles;
-        int s = 1;
-        while (s < 16 && k / (2 * s) >= 256 && 2.0 * s <= want * 1.41421356) s *= 2;
-        if (s > 1) return with_splits(64, n96 ? 96 : 64, 32, k, s);
-    }
-    int64_t tiles96 = (int64_t)((m + 63) / 64) * ((n + 95) / 96) * batch;
-    if (n96 && tiles96 <= cus) best.bn = 96;
     return best;
 }
+// Whether the split-operand kernel takes the product: 32-bit byte offsets inside a tile, room to count k past its end,
+// and at least 16 terms per sum (a shorter one is a rounding or two in fp32, which the split's own last roundings
+// exceed: with a single term the fp32 product is correctly rounded and the split's is not).
+bool s_takes(const Params &p, bool ta, bool tb) {
+    const int64_t ld = p.lda > p.ldb ? p.lda : p.ldb;
+    return !(ta && tb) && p.n >= 4 && p.k >= 16 && p.k < INT32_MAX - 4096 && ld < ((int64_t)1 << 22);
+}
+// Tile order of the grouped weight gradients: bands of 8 tile rows walked column by column when the group runs
+// unsplit (the workgroups one XCD runs together then share operand panels), row-major when it splits K.
+int group_band(int splits) { return splits == 1 ? 8 : 0; }
+}  // namespace
 
 // Thin products (one side at most 32: a classifier head's weight gradient, 9 x 768 over K = 4096 tokens) take the
 // 128 x 32 / 32 x 128 tiles. Products with fewer tiles than CUs (the classifier heads, small batches) split K into
@@ -531,99 +297,138 @@ Choice choose(int m, int n, int k, int batch, int cus) {
     return c;
 }
 
+// Short sums over few tiles on the tile-exact fp32 kernels: whole 64 x 96 (or 64 x 64) tiles, at most one per CU, and at
+// most five chunks of 32 k. Against the split-operand kernel (us, both ways timed back to back): 4096 x 384 at k 32 / 64
+// / 128 / 192 / 256 5.0 / 5.8 / 7.3 / 8.8 / 10.4 here and 6.1 / 7.6 / 8.7 / 9.6 / 10.3 there, 1024 x 256 4.2 / 4.4 / 5.5 /
+// 6.6 / 7.7 and 5.1 / 5.1 / 6.5 / 6.8 / 7.8; with more than a tile per CU the split kernel wins from k = 32 on (4096 x
+// 1536 11.1 and 10.6). Both operands K-contiguous take the chunks straight into LDS. Returns the tile width (0: the
+// product is not taken). A GELU epilogue's family is compiled in (0 none, 1 the reference's polynomials, 2 the pair of
+// stated error with the slope product).
+static int short_tile(const Params &p, bool ta, bool tb, int batch, int cus) {
+    const bool al = ((uintptr_t)p.a % 16 == 0) && ((uintptr_t)p.b % 16 == 0) && p.lda % 4 == 0 && p.ldb % 4 == 0 &&
+                    p.sa_outer % 4 == 0 && p.sa_inner % 4 == 0 && p.sb_outer % 4 == 0 && p.sb_inner % 4 == 0;
+    if (!al || (ta && tb) || p.k <= 0 || p.k > 160 || p.k % 32 || p.m % 64) return 0;
+    const int bn = p.n % 96 == 0 ? 96 : p.n % 64 == 0 ? 64 : 0;
+    if (!bn || (int64_t)(p.m / 64) * (p.n / bn) * batch > cus) return 0;
+    const int64_t ld = p.lda > p.ldb ? p.lda : p.ldb;
+    return ld * 96 < (int64_t)1 << 31 ? bn : 0;
+}
+template <int BN>
+static void launch_short(const Params &p, bool ta, bool tb, int batch, hipStream_t st) {
+    const dim3 grid((unsigned)((p.m / 64) * (p.n / BN) * batch));
+    const int gk = p.epi == EPI_GELU || p.epi == EPI_GELU_GRAD || p.epi == EPI_GELU_SLOPE ? 1
+                   : p.epi == EPI_NONE || p.epi == EPI_RELU                               ? 0
+                                                                                          : 2;
+    if (ta) {
+        hipLaunchKernelGGL((gx::k_gemm_x<64, BN, 32, true, false, 0>), grid, dim3(NT), 0, st, p);
+    } else if (tb) {
+        if (gk == 0) hipLaunchKernelGGL((gx::k_gemm_xd<64, BN, 32, 0>), grid, dim3(NT), 0, st, p);
+        else if (gk == 1) hipLaunchKernelGGL((gx::k_gemm_x<64, BN, 32, false, true, 1>), grid, dim3(NT), 0, st, p);
+        else hipLaunchKernelGGL((gx::k_gemm_xd<64, BN, 32, 2>), grid, dim3(NT), 0, st, p);
+    } else {
+        if (gk == 0) hipLaunchKernelGGL((gx::k_gemm_x<64, BN, 32, false, false, 0>), grid, dim3(NT), 0, st, p);
+        else if (gk == 1) hipLaunchKernelGGL((gx::k_gemm_x<64, BN, 32, false, false, 1>), grid, dim3(NT), 0, st, p);
+        else hipLaunchKernelGGL((gx::k_gemm_x<64, BN, 32, false, false, 2>), grid, dim3(NT), 0, st, p);
+    }
+}
+
+// The split-K reduce of one product.
+static om_status launch_reduce(om_ctx *ctx, const Params &p, hipStream_t st, const char *what) {
+    if (p.splits <= 1) return OM_OK;
+    const int64_t quads = (int64_t)p.m * (p.n / 4);
+    const dim3 grid(om::grid1d(quads > p.m ? quads : p.m, 256, 4096));
+#define OMG_R(S)                                                                      \
+    if (p.n % 4 == 0 && p.splits == S) {                                              \
+        hipLaunchKernelGGL(k_splitk_reduce_s<S>, grid, dim3(256), 0, st, p);          \
+        return OM_LAUNCH_CHECK(ctx, what);                                            \
+    }
+    OMG_R(2) OMG_R(3) OMG_R(4) OMG_R(5) OMG_R(6) OMG_R(7) OMG_R(8) OMG_R(12) OMG_R(16)
+#undef OMG_R
+    hipLaunchKernelGGL(k_splitk_reduce, dim3(om::grid1d((int64_t)p.m * p.n, 256, 4096)), dim3(256), 0, st, p);
+    return OM_LAUNCH_CHECK(ctx, what);
+}
+
 om_status launch_dense(om_ctx *ctx, Params p, bool ta, bool tb, int batch, const char *what, bool *colsum_fused,
                        int *mse_slots) {
     if (colsum_fused) *colsum_fused = false;
     if (mse_slots) *mse_slots = 0;
     if (p.m <= 0 || p.n <= 0 || batch <= 0) return OM_OK;
     p.batch = batch;
-    bool vec = ((uintptr_t)p.a % 16 == 0) && ((uintptr_t)p.b % 16 == 0) && p.lda % 4 == 0 && p.ldb % 4 == 0 &&
-               p.sa_outer % 4 == 0 && p.sa_inner % 4 == 0 && p.sb_outer % 4 == 0 && p.sb_inner % 4 == 0;
-    bool fast = vec && !(ta && tb) && p.k > 0 && p.m > 32 && p.n > 32 && p.m % 4 == 0 && p.n % 4 == 0 &&
-                p.k % 4 == 0;
-    // The slope product (EPI_MUL_AUX) takes the tiles of the GELU products of the context's mode, so that in either
-    // mode om_linear_bwd_dx_slope of the forward's slope and om_linear_bwd_dx_gelu give the same bits.
-    int fam = epi_family(p.epi);
-    if (fam == 3) fam = ctx->gelu_mode == OM_GELU_REFERENCE ? 1 : 2;
-    Choice c = p.k <= 0 ? Choice{64, 64, 1, 1, 16}
-                        : (fast ? choose_fast(p.m, p.n, p.k, batch, ta, tb, ctx->num_cus, fam)
-                                : choose(p.m, p.n, p.k, batch, ctx->num_cus));
-    if (fast && fam == 1) {  // only some tiles carry the reference's GELU polynomials
-        const bool ok = ((c.bkt == 32 || c.bkt == 33) && c.bm == 64 && (c.bn == 64 || c.bn == 96)) ||
-                        (c.bkt == 64 && c.bm == 64 && c.bn == 64);
-        if (!ok) c = with_splits(64, 64, 32, p.k, c.splits);
-    } else if (fast && fam == 2) {  // the fast pair and the slope product: the tiles of dispatch_x's list
-        const bool ok = (c.bkt == 32 && ((c.bm == 64 && (c.bn == 64 || c.bn == 96 || c.bn == 128)) ||
-                                         (c.bm == 128 && (c.bn == 64 || c.bn == 96 || c.bn == 128)))) ||
-                        (c.bkt == 33 && ((c.bm == 64 && c.bn == 96) || (c.bm == 128 && (c.bn == 96 || c.bn == 128))));
-        if (!ok) c = with_splits(64, 64, 32, p.k, c.splits);
+    p.xcd_remap = 1;
+    p.ws = nullptr;
+    const hipStream_t st = om::cur_stream(ctx);
+    // (a GELU gradient with a transposed A has no instance there; no caller asks for one)
+    const int bn = ta && p.epi != EPI_NONE && p.epi != EPI_RELU ? 0 : short_tile(p, ta, tb, batch, ctx->num_cus);
+    if (bn) {
+        p.splits = 1;
+        p.k_split = p.k;
+        const bool cs = p.db && ta && batch == 1;
+        if (!cs) p.db = nullptr;
+        p.colsum_ws = nullptr;
+        if (colsum_fused) *colsum_fused = cs;
+        if (p.mse_t && batch == 1) {
+            if (mse_slots) *mse_slots = (p.m / 64) * (p.n / bn) * 4;
+        } else {
+            p.mse_t = nullptr;
+            p.mse_unit = nullptr;
+            p.mse_part = nullptr;
+        }
+        if (bn == 96) launch_short<96>(p, ta, tb, batch, st);
+        else launch_short<64>(p, ta, tb, batch, st);
+        return OM_LAUNCH_CHECK(ctx, what);
     }
-    bool use_x = fast && !x_disabled() && x_fits(XTile{c.bm, c.bn, c.bkt}, p, c.splits, c.k_split);
-    if (fast && !use_x && c.bkt != 32) c = with_splits(c.bm, c.bn, 32, p.k, c.splits);  // guarded set: BK = 32
-    c.bkt = use_x ? c.bkt : 32;
+    if (s_takes(p, ta, tb)) {
+        const bool mask = p.mask != nullptr;
+        const SChoice c = choose_s(1, &p.m, &p.n, p.k, batch, ctx->num_cus, !mask);
+        p.splits = c.splits;
+        p.k_split = c.splits > 1 ? c.k_split : p.k;
+        const bool cs = p.db && ta && batch == 1;  // the bias gradient rides along with a weight gradient
+        if (!cs) p.db = nullptr;
+        p.colsum_ws = nullptr;
+        if (p.splits > 1) {
+            float *ws;
+            const uint64_t cbytes = cs ? (sizeof(double) * (uint64_t)p.splits * p.m + 255) / 256 * 256 : 0;
+            om_status s = om::scratch(ctx, cbytes + sizeof(float) * (uint64_t)p.splits * p.m * p.n, &ws);
+            if (s) return s;
+            p.colsum_ws = cs ? reinterpret_cast<double *>(ws) : nullptr;
+            p.ws = reinterpret_cast<float *>(reinterpret_cast<char *>(ws) + cbytes);
+        }
+        if (colsum_fused) *colsum_fused = cs;
+        const int64_t tiles = (int64_t)((p.m + c.c->bm - 1) / c.c->bm) * ((p.n + c.c->bn - 1) / c.c->bn);
+        const int64_t total = tiles * batch * p.splits;
+        OM_REQUIRE(ctx, total < ((int64_t)1 << 31), "%s: %lld workgroups", what, (long long)total);
+        if (p.mse_t && p.splits == 1 && batch == 1) {
+            if (mse_slots) *mse_slots = (int)(tiles * c.c->waves);
+        } else {
+            p.mse_t = nullptr;
+            p.mse_unit = nullptr;
+            p.mse_part = nullptr;
+        }
+        (ta ? launch_s_tn : tb ? launch_s_nt : launch_s_nn)(c.c->id, c.exact, p, (unsigned)total, st);
+        const om_status s = OM_LAUNCH_CHECK(ctx, what);
+        return s ? s : launch_reduce(ctx, p, st, what);
+    }
+    p.mse_t = nullptr;
+    p.mse_unit = nullptr;
+    p.mse_part = nullptr;
+    p.db = nullptr;
+    p.colsum_ws = nullptr;
+    const bool vec = ((uintptr_t)p.a % 16 == 0) && ((uintptr_t)p.b % 16 == 0) && p.lda % 4 == 0 && p.ldb % 4 == 0 &&
+                     p.sa_outer % 4 == 0 && p.sa_inner % 4 == 0 && p.sb_outer % 4 == 0 && p.sb_inner % 4 == 0;
+    const Choice c = p.k <= 0 ? Choice{64, 64, 1, 1, 16} : choose(p.m, p.n, p.k, batch, ctx->num_cus);
     p.splits = c.splits;
     p.k_split = c.splits > 1 ? c.k_split : (p.k > 0 ? p.k : 1);
-    p.ws = nullptr;
-    p.xcd_remap = 1;
-    // A fused bias gradient needs a tile-exact TN launch whose row groups divide the workgroup.
-    const bool cs = p.db && use_x && ta && !tb && batch == 1 && ((c.bkt & 1) ? 2 * NT : NT) % c.bm == 0;
-    if (!cs) {
-        p.db = nullptr;
-        p.colsum_ws = nullptr;
-    }
     if (p.splits > 1) {
-        float *ws;
-        const uint64_t cbytes = cs ? (sizeof(double) * (uint64_t)p.splits * p.m + 255) / 256 * 256 : 0;
-        om_status s = om::scratch(ctx, cbytes + sizeof(float) * (uint64_t)p.splits * p.m * p.n, &ws);
+        om_status s = om::scratch(ctx, sizeof(float) * (uint64_t)p.splits * p.m * p.n, &p.ws);
         if (s) return s;
-        p.colsum_ws = cs ? reinterpret_cast<double *>(ws) : nullptr;
-        p.ws = reinterpret_cast<float *>(reinterpret_cast<char *>(ws) + cbytes);
     }
-    if (colsum_fused) *colsum_fused = cs;
-    // The fused MSE needs the tile-exact epilogue over one split (one workgroup per tile, four wavefronts each).
-    const bool mse = p.mse_t && use_x && p.splits == 1 && batch == 1;
-    if (!mse) {
-        p.mse_t = nullptr;
-        p.mse_unit = nullptr;
-        p.mse_part = nullptr;
-    }
-    hipStream_t st = om::cur_stream(ctx);
-    bool launched = use_x && dispatch_x(XTile{c.bm, c.bn, c.bkt, c.dma}, p, batch, ta, tb, st, ctx->num_cus);
-    if (mse && launched && mse_slots) *mse_slots = (p.m / c.bm) * (p.n / c.bn) * 4;
-    if (launched) {
-    } else if (fast) {
-        if (c.bm == 128 && c.bn == 192) launch_fast<128, 192>(p, batch, ta, tb, st);
-        else if (c.bm == 192 && c.bn == 128) launch_fast<192, 128>(p, batch, ta, tb, st);
-        else if (c.bm == 128 && c.bn == 128) launch_fast<128, 128>(p, batch, ta, tb, st);
-        else if (c.bm == 128 && c.bn == 64) launch_fast<128, 64>(p, batch, ta, tb, st);
-        else if (c.bm == 64 && c.bn == 128) launch_fast<64, 128>(p, batch, ta, tb, st);
-        else if (c.bm == 64 && c.bn == 96) launch_fast<64, 96>(p, batch, ta, tb, st);
-        else if (c.bm == 96 && c.bn == 64) launch_fast<96, 64>(p, batch, ta, tb, st);
-        else launch_fast<64, 64>(p, batch, ta, tb, st);
-    } else {
-        if (c.bm == 128 && c.bn == 32) launch_general<128, 32>(p, batch, ta, tb, vec, st);
-        else if (c.bm == 32 && c.bn == 128) launch_general<32, 128>(p, batch, ta, tb, vec, st);
-        else launch_general<64, 64>(p, batch, ta, tb, vec, st);
-    }
-    om_status s = OM_LAUNCH_CHECK(ctx, what);
-    if (s || p.splits <= 1) return s;
-    if (p.n % 4 == 0 && (p.splits == 2 || p.splits == 4 || p.splits == 8 || p.splits == 16)) {
-        const int64_t quads = (int64_t)p.m * (p.n / 4);
-        const dim3 grid(om::grid1d(quads > p.m ? quads : p.m, 256, 4096));
-        if (p.splits == 2) hipLaunchKernelGGL(k_splitk_reduce_s<2>, grid, dim3(256), 0, st, p);
-        else if (p.splits == 4) hipLaunchKernelGGL(k_splitk_reduce_s<4>, grid, dim3(256), 0, st, p);
-        else if (p.splits == 8) hipLaunchKernelGGL(k_splitk_reduce_s<8>, grid, dim3(256), 0, st, p);
-        else hipLaunchKernelGGL(k_splitk_reduce_s<16>, grid, dim3(256), 0, st, p);
-    } else {
-        hipLaunchKernelGGL(k_splitk_reduce, dim3(om::grid1d((int64_t)p.m * p.n, 256, 4096)), dim3(256), 0, st,
-                           p);
-    }
-    return OM_LAUNCH_CHECK(ctx, what);
+    if (c.bm == 128 && c.bn == 32) launch_general<128, 32>(p, batch, ta, tb, vec, st);
+    else if (c.bm == 32 && c.bn == 128) launch_general<32, 128>(p, batch, ta, tb, vec, st);
+    else launch_general<64, 64>(p, batch, ta, tb, vec, st);
+    const om_status s = OM_LAUNCH_CHECK(ctx, what);
+    return s ? s : launch_reduce(ctx, p, st, what);
 }
 
-// Weight gradients dw_i (+)= g_i^T x_i of 2..kMaxGroup products sharing K = rows, with fused bias gradients, in one
-// tile-exact launch (and one split-K reduce). Returns false, launching nothing, when the products do not fit it:
-// then the caller runs them one by one. Each product's arithmetic is that of k_gemm_x at the group's tile and split.
 // Fills the column-sum items of g (prefix counts in wavefronts, one per column).
 static void set_column_sums(GroupParams &g, int ncs, const om_column_sum *cs) {
     g.ncs = ncs;
@@ -643,11 +448,10 @@ static om_status launch_group_reduce(om_ctx *ctx, const GroupParams &g, int spli
     OM_REQUIRE(ctx, qb + rb + cb < ((int64_t)1 << 31), "grouped reduce: %lld blocks", (long long)(qb + rb + cb));
     const dim3 grid((unsigned)(qb + rb + cb));
     const int c = (int)cb, r = (int)rb;
-    if (splits <= 1) hipLaunchKernelGGL(k_splitk_reduce_group<1>, grid, dim3(256), 0, stream, g, c, r);
-    else if (splits == 2) hipLaunchKernelGGL(k_splitk_reduce_group<2>, grid, dim3(256), 0, stream, g, c, r);
-    else if (splits == 4) hipLaunchKernelGGL(k_splitk_reduce_group<4>, grid, dim3(256), 0, stream, g, c, r);
-    else if (splits == 8) hipLaunchKernelGGL(k_splitk_reduce_group<8>, grid, dim3(256), 0, stream, g, c, r);
-    else hipLaunchKernelGGL(k_splitk_reduce_group<16>, grid, dim3(256), 0, stream, g, c, r);
+#define OMG_R(S) \
+    if (splits == S) hipLaunchKernelGGL(k_splitk_reduce_group<S>, grid, dim3(256), 0, stream, g, c, r);
+    OMG_R(1) OMG_R(2) OMG_R(3) OMG_R(4) OMG_R(5) OMG_R(6) OMG_R(7) OMG_R(8) OMG_R(12) OMG_R(16)
+#undef OMG_R
     return OM_LAUNCH_CHECK(ctx, "grouped reduce");
 }
 
@@ -656,41 +460,24 @@ static bool dw_groupable(const om_linear_dw &d) {
     auto al = [](const void *q) { return ((uintptr_t)q & 15) == 0; };
     return d.dw && d.out % 64 == 0 && d.in % 64 == 0 && al(d.g) && al(d.x) && al(d.dw);
 }
+// Weight gradients dw_i (+)= g_i^T x_i of 2..kMaxGroup products sharing K = rows, with fused bias gradients, in one
+// launch (and one split-K reduce), on the tile and split chosen for the group. Returns false, launching nothing, when
+// the products do not fit it: then the caller runs them one by one.
 static bool launch_dw_group(om_ctx *ctx, int count, const om_linear_dw *it, int rows, int ncs, const om_column_sum *cs,
                             om_status *st) {
     *st = OM_OK;
-    if (count < 2 || count > kMaxGroup || rows <= 0 || x_disabled()) return false;
-    bool n96 = true;
+    if (count < 2 || count > kMaxGroup || rows <= 0) return false;
+    int ms[kMaxGroup], ns[kMaxGroup];
     for (int i = 0; i < count; i++) {
         const om_linear_dw &d = it[i];
-        if (!dw_groupable(d)) return false;
-        if (d.in % 96) n96 = false;
-    }
-    // 64 x 64 tiles, split until there are about six workgroups per CU (measured on the four C3 weight gradients:
-    // 148 us at 64 x 64 with 4 splits against 152 us for the best 64 x 96 choice, 8 splits).
-    int bn = 64;
-    int64_t tiles = 0;
-    for (int i = 0; i < count; i++) tiles += (int64_t)(it[i].out / 64) * (it[i].in / bn);
-    int splits = 1;
-    while (splits < 16 && tiles * splits < 6 * (int64_t)ctx->num_cus && rows % (2 * splits * 32) == 0 &&
-           rows / (2 * splits) >= 256)
-        splits *= 2;
-    if (const char *gx = om::tuning_env("OM_GROUP_X")) {  // tuning builds: OM_GROUP_X="bn,splits" for this launch only
-        int fbn = 0, fsp = 0;
-        if (sscanf(gx, "%d,%d", &fbn, &fsp) == 2 && (fbn == 64 || (fbn == 96 && n96))) {
-            bn = fbn;
-            splits = fsp;
-        }
-    }
-    Choice forced{};
-    if (env_override(forced, rows)) {  // OM_GEMM_X="64,bn,32,splits" for measurements
-        if (forced.bm != 64 || forced.bkt != 32 || (forced.bn != 64 && forced.bn != 96) || (forced.bn == 96 && !n96))
+        if (!dw_groupable(d) || !s_takes(dense_params(d.out, d.in, rows, d.g, d.out, d.x, d.in, d.dw, d.in), true, false))
             return false;
-        bn = forced.bn;
-        splits = forced.splits;
+        ms[i] = d.out;
+        ns[i] = d.in;
     }
-    if (splits < 1 || (splits & (splits - 1)) || splits > 16 || rows % (splits * 32)) return false;
-    const int k_split = rows / splits;
+    const SChoice ch = choose_s(count, ms, ns, rows, 1, ctx->num_cus, true);
+    const int splits = ch.splits, bm = ch.c->bm, bn = ch.c->bn;
+    const int k_split = splits > 1 ? ch.k_split : rows;
     GroupParams g{};
     g.count = count;
     g.band = group_band(splits);
@@ -704,7 +491,6 @@ static bool launch_dw_group(om_ctx *ctx, int count, const om_linear_dw *it, int 
         p.batch = 1;
         p.splits = splits;
         p.k_split = k_split;
-        if (!x_fits(XTile{64, bn, 32}, p, splits, k_split)) return false;
         ws_floats += splits > 1 ? (uint64_t)splits * d.out * d.in : 0;
         cs_doubles += splits > 1 && d.db ? (uint64_t)splits * d.out : 0;
         g.p[i] = p;
@@ -731,7 +517,7 @@ static bool launch_dw_group(om_ctx *ctx, int count, const om_linear_dw *it, int 
     g.rstart[0] = 0;
     for (int i = 0; i < count; i++) {
         const Params &p = g.p[i];
-        g.start[i + 1] = g.start[i] + (p.m / 64) * (p.n / bn) * splits;
+        g.start[i + 1] = g.start[i] + ((p.m + bm - 1) / bm) * ((p.n + bn - 1) / bn) * splits;
         g.qstart[i + 1] = g.qstart[i] + (int64_t)p.m * (p.n / 4);
         g.rstart[i + 1] = g.rstart[i] + (splits > 1 && p.db ? p.m : 0);
     }
@@ -741,8 +527,7 @@ static bool launch_dw_group(om_ctx *ctx, int count, const om_linear_dw *it, int 
         g.rstart[i + 1] = g.rstart[count];
     }
     hipStream_t stream = om::cur_stream(ctx);
-    if (bn == 96) hipLaunchKernelGGL((gx::k_gemm_x_tn_group<64, 96, 32>), dim3(g.start[count]), dim3(NT), 0, stream, g);
-    else hipLaunchKernelGGL((gx::k_gemm_x_tn_group<64, 64, 32>), dim3(g.start[count]), dim3(NT), 0, stream, g);
+    launch_s_tn_group(ch.c->id, ch.exact, g, (unsigned)g.start[count], stream);
     *st = OM_LAUNCH_CHECK(ctx, "om_param_grads_group");
     if (*st) return true;
     if (splits == 1) {  // the products are complete: only the column sums are left
@@ -1541,9 +1326,9 @@ om_status om_linear_fwd_resid_mse(om_ctx *ctx, const float *x, const float *w, c
         om_status s = OM_LAUNCH_CHECK(ctx, "om_linear_fwd_resid_mse");
         return s ? s : om::mse_of(ctx, y, target, dpred_unit, loss, n, rb);
     }
-    // one partial per wavefront of every tile; no tile is smaller than 64 x 64
+    // one partial per wavefront of every tile; no tile is smaller than 64 x 64 or has more than eight
     float *scr;
-    om_status s = om::scratch2(ctx, sizeof(double) * 4 * (uint64_t)((rows + 63) / 64) * ((out + 63) / 64), &scr);
+    om_status s = om::scratch2(ctx, sizeof(double) * 8 * (uint64_t)((rows + 63) / 64) * ((out + 63) / 64), &scr);
     if (s) return s;
     omg::Params p = omg::dense_params(rows, out, in, x, in, w, in, y, out);
     p.bias = b;

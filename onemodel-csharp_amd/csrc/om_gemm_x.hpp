@@ -1,4 +1,6 @@
-// Tile-exact fp32 MFMA GEMM for gfx950: the kernel the training path's dense products run on.
+// Tile-exact fp32 MFMA GEMM for gfx950, for products that fill at most one round of 64-row tiles with short sums
+// (launch_short in om_gemm.hip holds the rule and its measurements): their time is the chain of loads, where splitting
+// operands costs more than the faster matrix instruction gives.
 //
 // Preconditions, checked on the host: every tile is full (m % BM == 0, n % BN == 0), every split's K range is a
 // multiple of BKT, operands are 16-byte aligned with leading dimensions (and batch strides) multiples of 4. With
@@ -569,163 +571,6 @@ __global__ void __launch_bounds__(NT) k_gemm_xd(Params p) {
     int tm, tn, zz;
     tile_coords(p, p.n / BN, p.m / BM, tm, tn, zz);
     gemm_xd_tile<BM, BN, BKT, GK>(p, tm, tn, zz);
-}
-
-// Weight gradients of several products in one launch (om_linear_bwd_dw_group): product i owns the workgroups
-// [start[i], start[i+1]) of the XCD-remapped grid, each a (tile, split) of its own Params, run by the same tile body.
-template <int BM, int BN, int BKT>
-__global__ void __launch_bounds__(NT) k_gemm_x_tn_group(GroupParams g) {
-    OM_LDS_POISON();
-    int lin = blockIdx.x;
-    const int total = gridDim.x;
-    if ((total & 7) == 0) lin = (lin & 7) * (total >> 3) + (lin >> 3);
-    int i = 0;
-#pragma unroll
-    for (int j = 1; j < kMaxGroup; j++)
-        if (j < g.count && lin >= g.start[j]) i = j;
-    const Params &p = g.p[i];
-    const int local = lin - g.start[i], tiles_n = p.n / BN, tiles_m = p.m / BM;
-    if (g.band > 0) {
-        // Within a split: bands of `band` tile rows (the last band may be shorter), each walked one tile column at a
-        // time with the band's rows fastest, so the workgroups that run together on one XCD share few operand slabs.
-        const int per = tiles_m * tiles_n, split = local / per, idx = local % per;
-        const int bh = g.band < tiles_m ? g.band : tiles_m;
-        const int band = idx / (bh * tiles_n), r0 = band * bh, rows = min(bh, tiles_m - r0);
-        const int within = idx - r0 * tiles_n;
-        gemm_x_tile<BM, BN, BKT, true, false, false>(p, r0 + within % rows, within / rows, split);
-        return;
-    }
-    const int rest = local / tiles_n;
-    gemm_x_tile<BM, BN, BKT, true, false, false>(p, rest % tiles_m, local % tiles_n, rest / tiles_m);
-}
-
-// The same tile with eight wavefronts: two groups of four (2 x 2 over the tile, as above) split each chunk's 16-k
-// blocks between them (group g takes blocks g, g+2, ...), so every SIMD runs two wavefronts of the tile and one's LDS
-// and barrier waits hide behind the other's MFMAs. At the end group 1 hands its partial sums to group 0 through LDS
-// and group 0 adds them (in that fixed order) and runs the epilogue. For products with about one tile per CU.
-template <int BM, int BN, int BKT, bool TA, bool TB, int GK = 0>
-__global__ void __launch_bounds__(2 * NT) k_gemm_x2(Params p) {
-    OM_LDS_POISON();
-    constexpr int NTH = 2 * NT;
-    constexpr bool AK = !TA, BKL = TB;
-    constexpr int TM = BM / 32, TN = BN / 32, NB = BKT / 16;
-    static_assert(NB % 2 == 0, "each group needs whole 16-k blocks");
-    using LA = Ld<BM, BKT, AK, NTH>;
-    using LB = Ld<BN, BKT, BKL, NTH>;
-    __shared__ __attribute__((aligned(16))) float Sh[2 * LA::LDSZ + 2 * LB::LDSZ];
-    static_assert(2 * (LA::LDSZ + LB::LDSZ) >= BM * BN, "the partial-sum exchange reuses the operand buffers");
-    float *As = Sh, *Bs = Sh + 2 * LA::LDSZ;
-
-    const int tiles_n = p.n / BN, tiles_m = p.m / BM;
-    int tm, tn, zz;
-    tile_coords(p, tiles_n, tiles_m, tm, tn, zz);
-    if (zz >= p.batch * p.splits) return;
-    const int z = zz / p.splits, split = zz % p.splits;
-    const int outer = z / p.batch_div, inner = z % p.batch_div;
-    const float *A = p.a + outer * p.sa_outer + inner * p.sa_inner;
-    const float *B = p.b + outer * p.sb_outer + inner * p.sb_inner;
-    const int m0 = tm * BM, n0 = tn * BN;
-    const int kbeg = split * p.k_split;
-    const int nk = (min(p.k, kbeg + p.k_split) - kbeg) / BKT;
-    const int lane = threadIdx.x & 63, wv = (threadIdx.x >> 6) & 3, kg = threadIdx.x >> 8;
-    const int l16 = lane & 15, kl = lane >> 4;
-    const int wm0 = (wv >> 1) * (BM / 2), wn0 = (wv & 1) * (BN / 2);
-
-    floatx4 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const LA la(A, p.lda, m0);
-    const LB lb(B, p.ldb, n0);
-    constexpr bool CS_OK = TA && (NTH % BM == 0) && (BKT % (NTH / BM) == 0);
-    ColSum<CS_OK ? BM : 64, BKT, NTH> cs;
-    const bool do_cs = CS_OK && p.db && tn == 0;
-    auto chunk = [&](const float *Ab, const float *Bb) {
-        if constexpr (CS_OK)
-            if (do_cs) cs.add(Ab);
-#pragma unroll
-        for (int blk = 0; blk < NB; blk += 2) {
-            float fa[4][TM], fb[4][TN];
-            read_frag<BM, BKT, TM, AK>(fa, Ab, blk + kg, wm0, l16, kl);
-            read_frag<BN, BKT, TN, BKL>(fb, Bb, blk + kg, wn0, l16, kl);
-#pragma unroll
-            for (int s = 0; s < 4; s++)
-#pragma unroll
-                for (int i = 0; i < TM; i++)
-#pragma unroll
-                    for (int j = 0; j < TN; j++)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[s][i], fb[s][j], acc[i][j], 0, 0, 0);
-        }
-    };
-    if (nk > 0) {
-        floatx4 ra0[LA::NV], rb0[LB::NV], ra1[LA::NV], rb1[LB::NV];
-        const int klast = kbeg + (nk - 1) * BKT;
-        float *A0 = As, *A1 = As + LA::LDSZ, *B0 = Bs, *B1 = Bs + LB::LDSZ;
-        la.fetch(ra0, kbeg);
-        lb.fetch(rb0, kbeg);
-        la.fetch(ra1, min(kbeg + BKT, klast));
-        lb.fetch(rb1, min(kbeg + BKT, klast));
-        la.put(ra0, A0);
-        lb.put(rb0, B0);
-        __syncthreads();
-        int t = 0;
-        for (; t + 2 < nk; t += 2) {  // both halves always run (clamped loads), see k_gemm_x
-            la.fetch(ra0, min(kbeg + (t + 2) * BKT, klast));
-            lb.fetch(rb0, min(kbeg + (t + 2) * BKT, klast));
-            __builtin_amdgcn_sched_barrier(0);
-            chunk(A0, B0);
-            la.put(ra1, A1);
-            lb.put(rb1, B1);
-            __syncthreads();
-            la.fetch(ra1, min(kbeg + (t + 3) * BKT, klast));
-            lb.fetch(rb1, min(kbeg + (t + 3) * BKT, klast));
-            __builtin_amdgcn_sched_barrier(0);
-            chunk(A1, B1);
-            la.put(ra0, A0);
-            lb.put(rb0, B0);
-            __syncthreads();
-        }
-        const float *Al = A0, *Bl = B0;
-        if (nk - t == 2) {
-            chunk(A0, B0);
-            la.put(ra1, A1);
-            lb.put(rb1, B1);
-            __syncthreads();
-            Al = A1;
-            Bl = B1;
-        }
-        chunk(Al, Bl);
-    }
-    if constexpr (CS_OK)
-        if (p.db && tn == 0) {
-            __syncthreads();
-            cs.finish(p, reinterpret_cast<double *>(Sh), m0, split);
-        }
-    // Group 1's partial sums -> LDS (the operand buffers, after everyone is done with them) -> group 0.
-    __syncthreads();
-    float *X = Sh;  // [4 waves][TM*TN*4][64 lanes]
-    constexpr int PER = TM * TN * 4;
-    if (kg == 1) {
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-#pragma unroll
-            for (int j = 0; j < TN; j++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) X[(wv * PER + (i * TN + j) * 4 + r) * 64 + lane] = acc[i][j][r];
-    }
-    __syncthreads();
-    if (kg == 1) return;
-#pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) acc[i][j][r] = acc[i][j][r] + X[(wv * PER + (i * TN + j) * 4 + r) * 64 + lane];
-
-    float *C = p.c + outer * p.sc_outer + inner * p.sc_inner;
-    const float *mask = p.mask ? p.mask + outer * p.mask_outer_stride : nullptr;
-    tile_epilogue<TM, TN, AK, BKL, GK>(p, acc, C, mask, m0, n0, wm0, wn0, l16, kl, split);
 }
 
 }  // namespace gx

@@ -1,0 +1,113 @@
+"""The split-operand product (csrc/om_gemm_s.hpp) at the sizes and values where it can go wrong: partial tiles in both
+directions, K tails and uneven k groups, the last partial quad of columns, split K with its reduce, odd leading
+dimensions, and operands the three-way bf16 split does not carry (infinities, NaN, values past the largest bf16, values
+whose low part underflows), against float64.
+
+Tolerance: the sequential-accumulation bound k 2^-24 |A||B| that test_gemm_parity holds the product to (the kernel's own
+rounding count is lower: one per 16 terms and six per 16 on sums 2^-8 as large).
+"""
+import numpy as np
+import pytest
+
+import gpu_util
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return gpu_util.Dev()
+
+
+def product(dev, ta, tb, A, B, m, n, k, ldc=None, c0=None, bias=None, acc=0):
+    a, b = dev.put(A), dev.put(B)
+    c = dev.put(c0) if c0 is not None else dev.empty((m, n), fill=np.nan)
+    dev.call("om_gemm", ta, tb, m, n, k, a, A.shape[1], b, B.shape[1], c, ldc or n,
+             dev.put(bias) if bias is not None else None, acc, None)
+    return dev.get(c)
+
+
+def operands(rng, ta, tb, m, n, k, pad=0):
+    A = rng.standard_normal((k, m + pad) if ta else (m, k + pad)).astype(np.float32)
+    B = rng.standard_normal((n, k + pad) if tb else (k, n + pad)).astype(np.float32)
+    A64 = (A[:, :m].T if ta else A[:, :k]).astype(np.float64)
+    B64 = (B[:, :k].T if tb else B[:, :n]).astype(np.float64)
+    return A, B, A64, B64
+
+
+LAYOUTS = [(0, 1), (0, 0), (1, 0)]
+SHAPES = [(1, 4, 16), (31, 5, 33), (33, 7, 47), (64, 65, 31), (65, 63, 127), (127, 97, 129), (129, 95, 161), (257, 130, 200),
+          (96, 255, 513), (70, 66, 4099), (1030, 390, 95), (2050, 258, 321), (4096, 99, 40)]
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", SHAPES)
+def test_edges(dev, ta, tb, m, n, k):
+    rng = np.random.default_rng(m + 31 * n + 1009 * k)
+    A, B, A64, B64 = operands(rng, ta, tb, m, n, k, pad=3)
+    bias = rng.standard_normal(n).astype(np.float32)
+    c0 = rng.standard_normal((m, n + 1)).astype(np.float32)
+    got = product(dev, ta, tb, A, B, m, n, k, ldc=n + 1, c0=c0.copy(), bias=bias, acc=1)
+    assert np.array_equal(got[:, n], c0[:, n])  # nothing past the last column
+    want = A64 @ B64 + bias + c0[:, :n]
+    bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + 2.0 ** -22 * (np.abs(bias) + np.abs(c0[:, :n]) + np.abs(want))
+    assert np.all(np.abs(got[:, :n] - want) <= bound)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(130, 70, 200), (512, 384, 384)])
+def test_values_the_split_does_not_carry(dev, ta, tb, m, n, k):
+    rng = np.random.default_rng(5)
+    A, B, A64, B64 = operands(rng, ta, tb, m, n, k)
+
+    def put(row, col, v):
+        A[(col, row) if ta else (row, col)] = v
+        A64[row, col] = v
+
+    put(3, 1, np.inf)
+    put(m - 1, k - 1, -np.inf)
+    put(40, k // 2, np.nan)
+    put(70, 9, 3.4e38)  # finite, past the largest bf16
+    # one row, and elsewhere one column, of values whose low parts underflow
+    for c in range(k):
+        put(100, c, A64[100, c] * 1e-36)
+    if tb:
+        B[20] *= np.float32(1e-30)
+    else:
+        B[:, 20] *= np.float32(1e-30)
+    B64 = (B.T if tb else B).astype(np.float64)
+    A64 = (A.T if ta else A).astype(np.float64)
+    # keep the large row's sums inside fp32: its partner values shrink by 2^-10 in every column
+    if tb:
+        B[:, 9] *= np.float32(2.0 ** -10)
+    else:
+        B[9] *= np.float32(2.0 ** -10)
+    B64 = (B.T if tb else B).astype(np.float64)
+    got = product(dev, ta, tb, A, B, m, n, k)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = A64 @ B64
+        bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + 2.0 ** -148 * k
+    fin = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert np.all(np.abs(got[fin] - want[fin]) <= bound[fin])
+
+
+@pytest.mark.parametrize("rows,sizes", [(999, [(128, 192), (64, 64)]), (4100, [(384, 384), (1152, 384), (384, 1536)]),
+                                        (96, [(64, 128), (192, 64), (128, 64), (64, 64)])])
+def test_grouped_weight_gradients(dev, rows, sizes):
+    rng = np.random.default_rng(rows)
+    items = (dev.pkg.om_linear_dw * len(sizes))()
+    keep, want = [], []
+    for it, (out, in_) in zip(items, sizes):
+        g, x = (rng.standard_normal((rows, s)).astype(np.float32) for s in (out, in_))
+        b = [dev.put(g), dev.put(x), dev.empty((out, in_), fill=np.nan), dev.empty((out,), fill=np.nan)]
+        keep.append(b)
+        it.g, it.x, it.dw, it.db = (t.data_ptr() for t in b)
+        it.in_, it.out, it.acc_dw, it.acc_db = in_, out, 0, 0
+        want.append((g.astype(np.float64), x.astype(np.float64)))
+    dev.call("om_linear_bwd_dw_group", len(sizes), items, rows)
+    for b, (g, x) in zip(keep, want):
+        assert np.all(np.abs(dev.get(b[2]) - g.T @ x) <= rows * 2.0 ** -24 * (np.abs(g).T @ np.abs(x)))
+        s = g.sum(0)
+        assert np.all(np.abs(dev.get(b[3]) - s) <= 2.0 ** -23 * np.abs(s) + 1e-12 * np.abs(g).sum(0))  # summed in double
