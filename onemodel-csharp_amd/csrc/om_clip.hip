@@ -22,30 +22,40 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kPer = 8;                                  // float4 groups per thread per chunk
 constexpr int64_t kChunk = (int64_t)kBlock * 4 * kPer;  // 8192 floats per workgroup
-constexpr int kMaxSeg = 32;                              // segments per launch (kernel-argument table)
+// Segments per launch (kernel-argument table, 2.6 KB). A launch that ends costs the next one its ramp: 28.4M gradients in
+// 66 unaligned segments took three launches of at most 32 with scalar loads (21 + 21 + 7 us), one of 66 takes 37 us.
+constexpr int kMaxSeg = 128;
 
 struct Segs {
     float *ptr[kMaxSeg];
     int64_t len[kMaxSeg];
-    int64_t first[kMaxSeg + 1];  // first chunk of each segment within this launch; first[n] = chunks in the launch
+    uint32_t first[kMaxSeg + 1];  // first chunk of each segment within this launch; first[n] = chunks in the launch
     int n;
 };
+// Segments start at any element: 16-byte accesses need 4-byte alignment only.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// The segment holding chunk c of the launch, the chunk's first element and its length.
-__device__ __forceinline__ float *chunk_of(const Segs &s, int64_t c, int64_t &len, bool &vec) {
-    int i = 0;
-    while (i + 1 < s.n && s.first[i + 1] <= c) i++;
-    float *g = s.ptr[i];
-    const int64_t base = (c - s.first[i]) * kChunk;
+// The segment holding chunk c of the launch (binary search: a scan of the table was a chain of up to 32 scalar loads
+// before a workgroup's first gradient load), the chunk's first element and its length.
+__device__ __forceinline__ float *chunk_of(const Segs &s, uint32_t c, int64_t &len) {
+    int i = 0, end = s.n;
+    while (end - i > 1) {
+        const int mid = (i + end) >> 1;
+        if (s.first[mid] <= c) i = mid;
+        else end = mid;
+    }
+    const int64_t base = (int64_t)(c - s.first[i]) * kChunk;
     const int64_t rest = s.len[i] - base;
     len = rest < kChunk ? rest : kChunk;
-    vec = ((uintptr_t)g & 15) == 0;
-    return g + base;
+    return s.ptr[i] + base;
 }
 
 // Four consecutive elements e..e+3 of a chunk (zeros past its end; a zero adds nothing to either norm).
-__device__ __forceinline__ float4 load4(const float *g, int64_t e, int64_t len, bool vec) {
-    if (vec && e + 4 <= len) return *reinterpret_cast<const float4 *>(g + e);
+__device__ __forceinline__ float4 load4(const float *g, int64_t e, int64_t len) {
+    if (e + 4 <= len) {
+        const f4u v = *reinterpret_cast<const f4u *>(g + e);
+        return make_float4(v[0], v[1], v[2], v[3]);
+    }
     float4 v;
     v.x = e < len ? g[e] : 0.0f;
     v.y = e + 1 < len ? g[e + 1] : 0.0f;
@@ -87,11 +97,10 @@ __global__ void __launch_bounds__(kBlock) k_norm_partial(Segs s, double *__restr
     OM_LDS_POISON();
     __shared__ double sh[kBlock / 64];
     int64_t len;
-    bool vec;
-    const float *g = chunk_of(s, blockIdx.x, len, vec);
+    const float *g = chunk_of(s, blockIdx.x, len);
     float4 v[kPer];
 #pragma unroll
-    for (int j = 0; j < kPer; j++) v[j] = load4(g, 4 * ((int64_t)j * kBlock + threadIdx.x), len, vec);
+    for (int j = 0; j < kPer; j++) v[j] = load4(g, 4 * ((int64_t)j * kBlock + threadIdx.x), len);
     double acc = 0.0;
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
@@ -138,18 +147,15 @@ __global__ void __launch_bounds__(kBlock) k_scale_segs(Segs s, const float *__re
     const float c = *coef;
     if (!(c < 1.0f)) return;
     int64_t len;
-    bool vec;
-    float *g = chunk_of(s, blockIdx.x, len, vec);
+    float *g = chunk_of(s, blockIdx.x, len);
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int64_t e = 4 * ((int64_t)j * kBlock + threadIdx.x);
-        if (vec && e + 4 <= len) {
-            float4 v = *reinterpret_cast<float4 *>(g + e);
-            v.x = v.x * c;
-            v.y = v.y * c;
-            v.z = v.z * c;
-            v.w = v.w * c;
-            *reinterpret_cast<float4 *>(g + e) = v;
+        if (e + 4 <= len) {
+            f4u v = *reinterpret_cast<f4u *>(g + e);
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = v[r] * c;
+            *reinterpret_cast<f4u *>(g + e) = v;
         } else {
             for (int r = 0; r < 4; r++)
                 if (e + r < len) g[e + r] = g[e + r] * c;
@@ -162,18 +168,15 @@ __device__ __forceinline__ float clamp_value(float v, float c) { return v > c ? 
 __global__ void __launch_bounds__(kBlock) k_clip_value(Segs s, float c) {
     OM_LDS_POISON();
     int64_t len;
-    bool vec;
-    float *g = chunk_of(s, blockIdx.x, len, vec);
+    float *g = chunk_of(s, blockIdx.x, len);
 #pragma unroll
     for (int j = 0; j < kPer; j++) {
         const int64_t e = 4 * ((int64_t)j * kBlock + threadIdx.x);
-        if (vec && e + 4 <= len) {
-            float4 v = *reinterpret_cast<float4 *>(g + e);
-            v.x = clamp_value(v.x, c);
-            v.y = clamp_value(v.y, c);
-            v.z = clamp_value(v.z, c);
-            v.w = clamp_value(v.w, c);
-            *reinterpret_cast<float4 *>(g + e) = v;
+        if (e + 4 <= len) {
+            f4u v = *reinterpret_cast<f4u *>(g + e);
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = clamp_value(v[r], c);
+            *reinterpret_cast<f4u *>(g + e) = v;
         } else {
             for (int r = 0; r < 4; r++)
                 if (e + r < len) g[e + r] = clamp_value(g[e + r], c);
@@ -191,7 +194,9 @@ om_status tables(om_ctx *ctx, const char *what, int count, float *const *grads, 
     for (int i = 0; i < count; i++) {
         OM_REQUIRE(ctx, lens[i] >= 0, "%s: segment %d has negative length", what, i);
         if (!grads[i] || lens[i] == 0) continue;  // a parameter without a gradient is skipped
-        if (out.empty() || out.back().n == kMaxSeg) {
+        const int64_t c = (lens[i] + kChunk - 1) / kChunk;
+        OM_REQUIRE(ctx, c < (int64_t)1 << 31, "%s: segments too large", what);
+        if (out.empty() || out.back().n == kMaxSeg || out.back().first[out.back().n] + c >= (int64_t)1 << 31) {
             out.emplace_back();
             out.back().n = 0;
             out.back().first[0] = 0;
@@ -199,12 +204,10 @@ om_status tables(om_ctx *ctx, const char *what, int count, float *const *grads, 
         Segs &s = out.back();
         s.ptr[s.n] = grads[i];
         s.len[s.n] = lens[i];
-        const int64_t c = (lens[i] + kChunk - 1) / kChunk;
-        s.first[s.n + 1] = s.first[s.n] + c;
+        s.first[s.n + 1] = s.first[s.n] + (uint32_t)c;
         s.n++;
         chunks += c;
     }
-    for (auto &s : out) OM_REQUIRE(ctx, s.first[s.n] < (int64_t)1 << 31, "%s: segments too large", what);
     return OM_OK;
 }
 

@@ -263,3 +263,25 @@ def test_tape_schedule_applies_before_each_step(pkg):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("count", [1, 2, 33, 128, 129, 300])
+def test_many_segments_at_odd_offsets(dev, count):
+    """Segment tables around one launch's 128 entries, every segment starting at its own alignment: the norm against
+    float64 and the in-place scaling exactly."""
+    rng = np.random.default_rng(count)
+    lens = [int(v) for v in rng.integers(1, 40, count)]
+    lens[count // 2] = 8192 * 2 + 3
+    flat = rng.standard_normal(sum(lens) + 1).astype(np.float32)
+    buf = dev.put(flat)
+    starts = 1 + np.concatenate([[0], np.cumsum(lens)[:-1]])
+    ptrs = (C.c_void_p * count)(*[buf.data_ptr() + 4 * int(s) for s in starts])
+    total, coef = dev.empty((1,)), dev.empty((1,))
+    dev.call("om_clip_grad_norm", count, ptrs, (C.c_int64 * count)(*lens), 0.5, 0, 1, total, coef)
+    norm = np.sqrt(np.sum(flat[1:].astype(np.float64) ** 2))
+    assert abs(float(dev.get(total)[0]) - norm) <= 2.0 ** -23 * norm
+    c = dev.get(coef)[0]
+    assert c == np.float32(0.5 / (norm + 1e-6)) or abs(float(c) - 0.5 / (norm + 1e-6)) <= 2.0 ** -23 * float(c)
+    want = flat.copy()
+    want[1:] = flat[1:] * c
+    assert np.array_equal(dev.get(buf), want)
