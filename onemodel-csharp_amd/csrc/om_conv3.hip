@@ -2,6 +2,8 @@
 // implicit GEMM on MFMA, the input staged through LDS once per tile (Ops.Conv2d, Ops.Layers.cs:279-336; ConvBackward,
 // BackwardNn.cs:317-402).
 //
+// Forward and dX run on split operands (om_conv3_s.hpp) for channels in sixteens and thirty-twos; what follows is the fp32
+// kernel for the rest, and dW.
 // Forward: y[n][co][p] = bias[co] + sum over taps t = (ky, kx) and channels ci of W[co][ci][t] x[n][ci][p + shift(t)]
 // (zero outside the image), optionally followed by ReLU. A workgroup takes 128 output pixels (flattened, so any width
 // works) of one image and a block of 32 or 64 output channels; per chunk of 8 input channels it stages the input rows
@@ -19,7 +21,7 @@
 // the result depends only on the shape.
 // Sums run in another order than the reference's im2col GEMM; they are fp32 sums of the same products (1e-5 scaled
 // error, tested).
-#include "om_internal.hpp"
+#include "om_conv3_s.hpp"
 
 namespace {
 
@@ -639,6 +641,81 @@ int stage_ns(int chans, int W, int R) {
     return 0;
 }
 
+// The split sums of a convolution: bias, ReLU, and the pool when it can ride along.
+om_status sum_splits(om_ctx *ctx, const float *ws, int nsplit, int N, int H, int W, int Cout, const float *bias, float *y,
+                     int acc, bool relu, const Conv3Pool *pool, bool *pooled) {
+    const int P = H * W;
+    const int64_t total = (int64_t)N * Cout * P;
+    if (pool && relu && !acc && pooled) {  // the sum, the ReLU and the max pool in one pass
+        const int64_t npool = (int64_t)N * Cout * (H / pool->kh) * (W / pool->kw);
+        hipLaunchKernelGGL(k_conv3_sum_pool, dim3(om::grid1d(npool, 256, 4096)), dim3(256), 0, ctx->stream, ws, nsplit,
+                           total, H, W, Cout, bias, y, pool->y, pool->idx, pool->kh, pool->kw, npool);
+        *pooled = true;
+    } else {
+        hipLaunchKernelGGL(k_conv3_sum, dim3(om::grid1d(total, 256, 4096)), dim3(256), 0, ctx->stream, ws, nsplit,
+                           total, P, Cout, bias, y, acc, relu ? 1 : 0);
+    }
+    return OM_LAUNCH_CHECK(ctx, "conv2d split sum");
+}
+
+// The split-operand kernel (om_conv3_s.hpp): input channels in sixteens, output channels in thirty-twos, any width whose
+// staged rows fit the LDS. Blocks of 64 output channels halve the input's staging; those of 32 need half the weights' LDS,
+// for rows too wide otherwise. Eight wavefronts (256 pixels) or four, and runs of input channels whose partial sums a
+// second pass adds, as the fp32 kernel's are: the least rounds of workgroups over the CUs times chunks, a chunk of eight
+// wavefronts costing 4 (measured 7.5 us), of four 3, and the second pass 4. Measured against the fp32 kernel (us): 32 x 64
+// x 28 x 28 37.7 -> 27.4, 64 x 256 -> 512 channels at 8 x 8 160 -> 95, 2 x 64 at 112 x 112 34.8 -> 27.1, 1 x 64 at 28 x 28
+// 12.4 -> 10.2, 2 x 32 -> 64 at 32 x 280 35.5 -> 22.6. With one or two chunks of wide rows on a quarter of the CUs the
+// first chunk's loads are not hidden and the fp32 kernel's smaller tiles keep the lead (1 x 32 at 32 x 224: 11.4 against
+// 16.2 us; past 256 columns the latter's staging falls apart, 39 against 17 us): those stay there. The dearest shape that
+// does not: 16 x 128 -> 32 channels at 32 x 192, 384 workgroups on 256 CUs, 77 -> 84 us.
+bool split_conv(om_ctx *ctx, const float *x, const float *w, const float *bias, float *y, int N, int Cin, int H, int W,
+                int Cout, int acc, om_status *st, bool flip, bool relu, const Conv3Pool *pool, bool *pooled) {
+    const int P = H * W;
+    if (Cin % 16 || Cout % 32 || (int64_t)H * W > 1 << 26 || (int64_t)N * Cin * P > INT32_MAX ||
+        (int64_t)N * Cout * P > INT32_MAX || (int64_t)Cout * 9 * Cin > INT32_MAX)
+        return false;
+    const int chunks = Cin / 16;
+    oc3::Args a{x, w, bias, y, nullptr, Cin, Cout, H, W, 0, 0, N, 1, chunks, acc, 0};
+    int CB = 0, NW = 0, units = 0;
+    int64_t grid_n = 0, best = INT64_MAX;
+    for (int cb = Cout % 64 == 0 ? 2 : 1; cb && !NW; cb--)
+        for (int nw = 8; nw >= 4; nw -= 4) {
+            const int R = (W - 1 + 32 * nw - 1) / W + 3, u = (R * (W + 2) * 4 + 64 * nw - 1) / (64 * nw);
+            if (u > 12 || oc3::lds_bytes(R, W, cb) > 160 << 10) continue;
+            const int nt = (P + 32 * nw - 1) / (32 * nw);
+            const int64_t tiles = (int64_t)nt * (Cout / (32 * cb)) * N;
+            for (int ns = 1; ns <= chunks && (ns == 1 || tiles * (ns - 1) < ctx->num_cus); ns++) {
+                const int cps = (chunks + ns - 1) / ns, n = (chunks + cps - 1) / cps;
+                const int64_t cost =
+                    (tiles * n + ctx->num_cus - 1) / ctx->num_cus * cps * (nw == 8 ? 4 : 3) + (n > 1 ? 4 : 0);
+                if (cost >= best || tiles * n >= (int64_t)1 << 31) continue;
+                best = cost;
+                CB = cb, NW = nw, units = u, grid_n = tiles * n;
+                a.R = R, a.ntile = nt, a.nsplit = n, a.cps = cps;
+            }
+        }
+    if (!NW || (chunks <= 2 && units > 6 && W % 4 == 0 && W <= 256 && grid_n * 4 <= ctx->num_cus)) return false;
+    const int NU = units <= 4 ? 4 : units <= 6 ? 6 : units <= 8 ? 8 : 12, lds = oc3::lds_bytes(a.R, W, CB);
+    if (a.nsplit > 1) {
+        *st = om::scratch2(ctx, sizeof(float) * (uint64_t)a.nsplit * N * Cout * P, &a.ws);
+        if (*st) return true;
+    }
+    a.relu = relu && a.nsplit == 1;
+    const dim3 grid((unsigned)grid_n), block(64 * NW);
+#define OMC3S(CB_, NW_, NU_)                                                                              \
+    if (CB == CB_ && NW == NW_ && NU == NU_) {                                                            \
+        if (flip) hipLaunchKernelGGL((oc3::k_conv3_s<CB_, NW_, NU_, true>), grid, block, lds, ctx->stream, a);  \
+        else hipLaunchKernelGGL((oc3::k_conv3_s<CB_, NW_, NU_, false>), grid, block, lds, ctx->stream, a);      \
+    }
+#define OMC3N(CB_, NW_) OMC3S(CB_, NW_, 4) OMC3S(CB_, NW_, 6) OMC3S(CB_, NW_, 8) OMC3S(CB_, NW_, 12)
+    OMC3N(1, 4) OMC3N(1, 8) OMC3N(2, 4) OMC3N(2, 8)
+#undef OMC3N
+#undef OMC3S
+    *st = OM_LAUNCH_CHECK(ctx, flip ? "om_conv2d_bwd dx" : "om_conv2d_fwd");
+    if (!*st && a.nsplit > 1) *st = sum_splits(ctx, a.ws, a.nsplit, N, H, W, Cout, bias, y, acc, relu, pool, pooled);
+    return true;
+}
+
 }  // namespace
 
 // The 3x3 / stride 1 / padding 1 paths; each returns false (launching nothing) when the shape is not one it takes.
@@ -677,6 +754,7 @@ bool om_conv3_fwd(om_ctx *ctx, const float *x, const float *w, const float *bias
         *st = OM_LAUNCH_CHECK(ctx, "om_conv2d_fwd");
         return true;
     }
+    if (split_conv(ctx, x, w, bias, y, N, Cin, H, W, Cout, acc, st, flip_weights, relu, pool, pooled)) return true;
     if (Cin % kFwdCk || Cout % 32 || W % 4 || (int64_t)N * Cin * P > INT32_MAX || (int64_t)N * Cout * P > INT32_MAX ||
         (int64_t)Cout * 9 * Cin > INT32_MAX)
         return false;
@@ -720,16 +798,8 @@ bool om_conv3_fwd(om_ctx *ctx, const float *x, const float *w, const float *bias
     OMC3(64, 1) OMC3(64, 2) OMC3(64, 3) OMC3(64, 4) OMC3(64, 6) OMC3(64, 8)
     OMC3(32, 1) OMC3(32, 2) OMC3(32, 3) OMC3(32, 4) OMC3(32, 6) OMC3(32, 8)
 #undef OMC3
-    if (nsplit > 1 && pool && relu && !acc && pooled) {  // the sum, the ReLU and the max pool in one pass
-        const int64_t npool = (int64_t)N * Cout * (H / pool->kh) * (W / pool->kw);
-        hipLaunchKernelGGL(k_conv3_sum_pool, dim3(om::grid1d(npool, 256, 4096)), dim3(256), 0, ctx->stream, ws, nsplit,
-                           total, H, W, Cout, bias, y, pool->y, pool->idx, pool->kh, pool->kw, npool);
-        *pooled = true;
-    } else if (nsplit > 1) {
-        hipLaunchKernelGGL(k_conv3_sum, dim3(om::grid1d(total, 256, 4096)), dim3(256), 0, ctx->stream, ws, nsplit,
-                           total, P, Cout, bias, y, acc, relu ? 1 : 0);
-    }
     *st = OM_LAUNCH_CHECK(ctx, flip_weights ? "om_conv2d_bwd dx" : "om_conv2d_fwd");
+    if (!*st && nsplit > 1) *st = sum_splits(ctx, ws, nsplit, N, H, W, Cout, bias, y, acc, relu, pool, pooled);
     return true;
 }
 

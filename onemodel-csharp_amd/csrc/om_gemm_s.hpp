@@ -29,53 +29,12 @@
 #pragma once
 
 #include "om_gemm_core.hpp"
+#include "om_split.hpp"
 
 namespace omg {
 namespace gs {
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-// Global accesses of operands whose rows need not be 16-byte aligned (the hardware takes 4-byte alignment).
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
-
-// Two fp32 values split into packed bf16 pairs, each part rounded to nearest. (v_dot2_f32_bf16 would give a residual in
-// one instruction, but it shares the matrix pipe: beside an MFMA it costs 16 cycles, the unpack and subtraction 8.)
-__device__ __forceinline__ uint32_t pack2(float x0, float x1) {
-    const bf16x2 v = {(__bf16)x0, (__bf16)x1};
-    return __builtin_bit_cast(uint32_t, v);
-}
-__device__ __forceinline__ void split2(float x0, float x1, uint32_t &h, uint32_t &m, uint32_t &l) {
-    h = pack2(x0, x1);
-    asm("" : "+v"(h));  // else the compiler converts x0 a second time instead of shifting h
-    const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xFFFF0000u);
-    m = pack2(r0, r1);
-    asm("" : "+v"(m));
-    l = pack2(r0 - __uint_as_float(m << 16), r1 - __uint_as_float(m & 0xFFFF0000u));
-}
-
-// One lane's eight values of a fragment (16 k), as three MFMA operands.
-struct Frag {
-    u32x4 p[3];
-    // Values 4 q .. 4 q + 3.
-    __device__ __forceinline__ void set4(int q, const float *x) {
-        uint32_t h, m, l;
-        split2(x[0], x[1], h, m, l);
-        p[0][2 * q] = h;
-        p[1][2 * q] = m;
-        p[2][2 * q] = l;
-        split2(x[2], x[3], h, m, l);
-        p[0][2 * q + 1] = h;
-        p[1][2 * q + 1] = m;
-        p[2][2 * q + 1] = l;
-    }
-};
-__device__ __forceinline__ floatx16 mma(u32x4 a, u32x4 b, floatx16 c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
+using namespace oms;
 
 // k of element e (0 .. 15) in lane group g, relative to its 32-step; elements 8 h .. 8 h + 7 are MFMA h's.
 __device__ __forceinline__ int kof(int g, int e) { return 8 * (e >> 2) + 4 * g + (e & 3); }
@@ -391,15 +350,7 @@ __device__ __forceinline__ void tile(const Params &p, int tm, int tn, int zz) {
 #pragma unroll
         for (int q = 0; q < 3; q++) f[q] = *reinterpret_cast<const u32x4 *>(cur + j * 6144 + q * 1024 + roff[j & 1][h]);
     };
-    auto mm = [&](const u32x4(&f)[3], const Frag &a, int j) {
-        // the small terms (B plane, A plane) mm, lh, hl, mh, hm, then hh
-        low[j] = mma(f[1], a.p[1], low[j]);
-        low[j] = mma(f[2], a.p[0], low[j]);
-        low[j] = mma(f[0], a.p[2], low[j]);
-        low[j] = mma(f[1], a.p[0], low[j]);
-        low[j] = mma(f[0], a.p[1], low[j]);
-        acc[j] = mma(f[0], a.p[0], acc[j]);
-    };
+    auto mm = [&](const u32x4(&f)[3], const Frag &a, int j) { mma6(f, a.p, acc[j], low[j]); };
     // Quad w of A into its half's fragment; `have` false (a k group without this step) gives zeros.
     auto split_a = [&](float (&x)[4], int w, bool have) {
         if (EDGE && KG > 1) {
@@ -496,19 +447,14 @@ __device__ __forceinline__ void tile(const Params &p, int tm, int tn, int zz) {
         __syncthreads();
     }
 
-    // Sums the split could not carry: non-finite, or so small that low parts may have underflowed.
     unsigned big = 0, small = 0xFFFFFFFFu;
 #pragma unroll
     for (int j = 0; j < TN; j++) {
         acc[j] += low[j];
 #pragma unroll
-        for (int e = 0; e < 16; e++) {
-            const unsigned u = __float_as_uint(acc[j][e]) & 0x7FFFFFFFu;
-            big = u > big ? u : big;
-            small = u - 1u < small ? u - 1u : small;  // zero becomes the largest: exact zeros are fine
-        }
+        for (int e = 0; e < 16; e++) note(acc[j][e], big, small);
     }
-    if (__any(big >= 0x7F800000u || small < 0x12800000u - 1u)) {  // 2^-90
+    if (beyond(big, small)) {
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             // column of the lane's LDS row, as the loads and the epilogue place it

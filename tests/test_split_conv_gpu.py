@@ -1,0 +1,88 @@
+"""The split-operand 3x3 convolution (csrc/om_conv3_s.hpp) at the sizes and values where it can go wrong: widths that are
+no multiple of 4, partial pixel tiles, both channel blocks, one chunk of channels and split channels, accumulation, and
+operands the three-way bf16 split does not carry, against float64 over the zero-padded input.
+
+Tolerance: the sequential-accumulation bound k 2^-24 sum |w||x| over the k = 9 Cin terms (the kernel's own rounding count
+is lower: one per 16 terms and six per 16 on sums 2^-8 as large), and a rounding of each later addition.
+"""
+import numpy as np
+import pytest
+
+import gpu_util
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def dev():
+    return gpu_util.Dev()
+
+
+def conv64(x, w):
+    """3x3 / stride 1 / padding 1 in float64: sum over taps of w[:, :, t] times the shifted, zero-padded input."""
+    n, ci, h, wd = x.shape
+    xp = np.zeros((n, ci, h + 2, wd + 2))
+    xp[:, :, 1:-1, 1:-1] = x
+    y = np.zeros((n, w.shape[0], h * wd))
+    for ky in range(3):
+        for kx in range(3):
+            y += w[:, :, ky, kx].astype(np.float64) @ xp[:, :, ky:ky + h, kx:kx + wd].reshape(n, ci, -1)
+    return y.reshape(n, -1, h, wd)
+
+
+def turned(w):
+    return np.ascontiguousarray(w[:, :, ::-1, ::-1].transpose(1, 0, 2, 3))
+
+
+# (images, Cin, Cout, H, W): dX exchanges the channels
+SHAPES = [(1, 32, 32, 1, 1), (1, 32, 64, 3, 5), (2, 64, 32, 7, 7), (3, 96, 64, 5, 33), (1, 512, 64, 2, 3), (2, 32, 96, 19, 27),
+          (40, 64, 64, 15, 17), (9, 32, 160, 31, 33), (300, 32, 32, 3, 3), (2, 32, 64, 4, 185), (1, 64, 32, 3, 189),
+          (1, 32, 64, 90, 62)]
+
+
+@pytest.mark.parametrize("N,Cin,Cout,H,W", SHAPES)
+def test_edges(dev, N, Cin, Cout, H, W):
+    rng = np.random.default_rng(N + 31 * Cin + 1009 * Cout + 7 * W)
+    x = rng.standard_normal((N, Cin, H, W)).astype(np.float32)
+    w = rng.standard_normal((Cout, Cin, 3, 3)).astype(np.float32)
+    b = rng.standard_normal(Cout).astype(np.float32)
+    g = rng.standard_normal((N, Cout, H, W)).astype(np.float32)
+    X, Wd, B, G = dev.put(x), dev.put(w), dev.put(b), dev.put(g)
+    Y, R = dev.empty(g.shape, fill=np.nan), dev.empty(g.shape, fill=np.nan)
+    dev.call("om_conv2d_fwd", X, Wd, B, Y, N, Cin, H, W, Cout, 3, 3, 1, 1)
+    want = conv64(x, w) + b[:, None, None]
+    bound = 9 * Cin * 2.0 ** -24 * conv64(np.abs(x), np.abs(w)) + 2.0 ** -22 * (np.abs(want) + np.abs(b)[:, None, None])
+    y = dev.get(Y)
+    assert np.all(np.abs(y - want) <= bound)
+    dev.call("om_conv2d_relu_fwd", X, Wd, B, R, N, Cin, H, W, Cout, 3, 3, 1, 1)
+    assert np.array_equal(dev.get(R), np.where(y > 0, y, np.float32(0)))
+    dx0 = rng.standard_normal(x.shape).astype(np.float32)
+    DX, DW, DB = dev.put(dx0.copy()), dev.empty(w.shape), dev.empty(b.shape)
+    dev.call("om_conv2d_bwd", G, X, Wd, DX, DW, DB, N, Cin, H, W, Cout, 3, 3, 1, 1, 1, 0)
+    want = conv64(g, turned(w)) + dx0
+    bound = 9 * Cout * 2.0 ** -24 * conv64(np.abs(g), turned(np.abs(w))) + 2.0 ** -22 * (np.abs(want) + np.abs(dx0))
+    assert np.all(np.abs(dev.get(DX) - want) <= bound)
+
+
+@pytest.mark.parametrize("N,C,H,W", [(6, 32, 17, 19), (1, 64, 6, 9)])
+def test_values_the_split_does_not_carry(dev, N, C, H, W):
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    w = rng.standard_normal((C, C, 3, 3)).astype(np.float32) * np.float32(2.0 ** -8)
+    x[0, 1, 0, 0], x[0, 2, 3, W - 1], x[0, 3, 5, 2], x[0, 4, 3, 5] = np.inf, -np.inf, np.nan, 3.4e38
+    w[7, 5, 2, 2] = np.inf  # times the zeros around the image: NaN along two edges, as the padded sum has it
+    w[9] *= np.float32(1e-36)
+    X, Wd, B, Y = dev.put(x), dev.put(w), dev.put(np.zeros(C, np.float32)), dev.empty(x.shape, fill=0)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for flip in (False, True):
+            if flip:
+                dev.call("om_conv2d_bwd", X, X, Wd, Y, dev.empty(w.shape), dev.empty((C,)), N, C, H, W, C, 3, 3, 1, 1, 0, 0)
+            else:
+                dev.call("om_conv2d_fwd", X, Wd, B, Y, N, C, H, W, C, 3, 3, 1, 1)
+            wf = turned(w) if flip else w
+            want = conv64(x, wf)
+            bound = 9 * C * (2.0 ** -24 * conv64(np.abs(x), np.abs(wf)) + 2.0 ** -148)
+            got, fin = dev.get(Y), np.isfinite(want)
+            assert np.array_equal(np.isnan(got), np.isnan(want))
+            assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+            assert np.all(np.abs(got[fin] - want[fin]) <= bound[fin])
