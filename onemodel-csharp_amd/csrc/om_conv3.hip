@@ -2,8 +2,8 @@
 // implicit GEMM on MFMA, the input staged through LDS once per tile (Ops.Conv2d, Ops.Layers.cs:279-336; ConvBackward,
 // BackwardNn.cs:317-402).
 //
-// Forward and dX run on split operands (om_conv3_s.hpp) for channels in sixteens and thirty-twos; what follows is the fp32
-// kernel for the rest, and dW.
+// Forward and dX run on split operands (om_conv3_s.hpp) for channels in sixteens and thirty-twos, and dW (om_conv3_dw_s.hpp)
+// where the width suits it; what follows are the fp32 kernels for the rest.
 // Forward: y[n][co][p] = bias[co] + sum over taps t = (ky, kx) and channels ci of W[co][ci][t] x[n][ci][p + shift(t)]
 // (zero outside the image), optionally followed by ReLU. A workgroup takes 128 output pixels (flattened, so any width
 // works) of one image and a block of 32 or 64 output channels; per chunk of 8 input channels it stages the input rows
@@ -21,6 +21,9 @@
 // the result depends only on the shape.
 // Sums run in another order than the reference's im2col GEMM; they are fp32 sums of the same products (1e-5 scaled
 // error, tested).
+#include <algorithm>
+
+#include "om_conv3_dw_s.hpp"
 #include "om_conv3_s.hpp"
 
 namespace {
@@ -716,6 +719,56 @@ bool split_conv(om_ctx *ctx, const float *x, const float *w, const float *bias, 
     return true;
 }
 
+// The slots' sums of a weight gradient (and its bias gradient).
+void reduce_dw(om_ctx *ctx, const float *part, int slots, int Cout, int Cin, float *dw, int acc, const double *dbp,
+               float *db) {
+    const int64_t total = (int64_t)Cout * 9 * Cin;
+    const unsigned rb = (unsigned)((total + 63) / 64 + (db ? (Cout + 63) / 64 : 0));
+    if (slots >= 256 && rb < (unsigned)ctx->num_cus)
+        hipLaunchKernelGGL(k_conv3_dw_reduce<16>, dim3(rb), dim3(1024), 0, ctx->stream, part, slots, Cout, Cin, dw, acc,
+                           dbp, db);
+    else
+        hipLaunchKernelGGL(k_conv3_dw_reduce<4>, dim3(rb), dim3(256), 0, ctx->stream, part, slots, Cout, Cin, dw, acc,
+                           dbp, db);
+}
+
+// The split-operand weight gradient (om_conv3_dw_s.hpp): input channels in thirty-twos, output channels in sixty-fours, about
+// two workgroups per CU and at least two items per slot. It takes the widths that are no multiple of 4, which the fp32
+// kernel below cannot stage and the general one ran, and widths from 112 on. Measured with the reduce (us, before and
+// after): 32 x 128 -> 128 channels at 27 x 27 202 -> 96, 8 x 64 at 57 x 57 76 -> 42, 2 x 32 -> 64 at 33 x 97 49 -> 20, 16 x 32
+// -> 64 at 15 x 17 28 -> 19, 4 x 32 -> 64 at 32 x 200 58 -> 27, 8 x 64 at 112 x 112 100 -> 90. At other multiples of 4 its
+// staging, which nothing hides but the CU's other workgroup, costs what the matrix cores save (32 x 64 at 56 x 56 88 against
+// 94, 28 x 28 37 against 41, 32 x 32 -> 64 at 16 x 64 28 against 27): the fp32 kernel keeps them. Below 4000 pixels too few
+// slots run (32 x 7 x 7 17.6 against 19.3, 1 x 9 x 9 15.5 against 23): the general kernel keeps those.
+bool split_dw(om_ctx *ctx, const float *g, const float *x, float *dw, float *db, int N, int Cin, int H, int W, int Cout,
+              int acc, om_status *st) {
+    const int64_t P = (int64_t)H * W;
+    if ((W % 4 == 0 && W < 112) || N * P < 4000) return false;
+    if (Cin % oc3w::kCi || Cout % oc3w::kCo || P > 1 << 26 || (int64_t)N * Cout * P > INT32_MAX ||
+        (int64_t)N * Cin * P > INT32_MAX)
+        return false;
+    int RB, SG, bands, segs;
+    oc3w::geometry(H, W, RB, SG, bands, segs);
+    const int blocks = (Cout / oc3w::kCo) * (Cin / oc3w::kCi);
+    if ((int64_t)N * bands * segs > INT32_MAX / 2) return false;
+    const int items = N * bands * segs;
+    const int want = std::max(1, std::min((2 * ctx->num_cus + blocks - 1) / blocks, items / 2));
+    const int per = (items + want - 1) / want, slots = (items + per - 1) / per;
+    const uint64_t pbytes = (sizeof(float) * (uint64_t)slots * Cout * 9 * Cin + 255) / 256 * 256;
+    float *part;
+    *st = om::scratch(ctx, pbytes + (db ? sizeof(double) * (uint64_t)slots * Cout : 0), &part);
+    if (*st) return true;
+    double *dbp = db ? reinterpret_cast<double *>(reinterpret_cast<char *>(part) + pbytes) : nullptr;
+    const oc3w::Args a{g, x, part, dbp, Cin, Cout, H, W, RB, SG, bands, segs, items, per};
+    const dim3 grid((unsigned)((int64_t)slots * blocks)), block(oc3w::kThreads);
+    const int lds = oc3w::lds_bytes(RB, SG);
+    if (W >= 4) hipLaunchKernelGGL(oc3w::k_conv3_dw_s<true>, grid, block, lds, ctx->stream, a);
+    else hipLaunchKernelGGL(oc3w::k_conv3_dw_s<false>, grid, block, lds, ctx->stream, a);
+    reduce_dw(ctx, part, slots, Cout, Cin, dw, acc, dbp, db);
+    *st = OM_LAUNCH_CHECK(ctx, "om_conv2d_bwd dw");
+    return true;
+}
+
 }  // namespace
 
 // The 3x3 / stride 1 / padding 1 paths; each returns false (launching nothing) when the shape is not one it takes.
@@ -829,6 +882,7 @@ bool om_conv3_dw(om_ctx *ctx, const float *g, const float *x, float *dw, float *
         *st = OM_LAUNCH_CHECK(ctx, "om_conv2d_bwd dw");
         return true;
     }
+    if (split_dw(ctx, g, x, dw, db, N, Cin, H, W, Cout, acc, st)) return true;
     if (Cin % kDwCi || Cout % kDwCo || W % 4 || (int64_t)N * Cout * P > INT32_MAX || (int64_t)N * Cin * P > INT32_MAX)
         return false;
     int R, ps;
@@ -855,14 +909,7 @@ bool om_conv3_dw(om_ctx *ctx, const float *g, const float *x, float *dw, float *
                            nchunks, items, per, dbp);
     OMW3(1) OMW3(2) OMW3(3) OMW3(4) OMW3(6) OMW3(8)
 #undef OMW3
-    const int64_t total = (int64_t)Cout * 9 * Cin;
-    const unsigned rb = (unsigned)((total + 63) / 64 + (db ? (Cout + 63) / 64 : 0));
-    if (slots >= 256 && rb < (unsigned)ctx->num_cus)
-        hipLaunchKernelGGL(k_conv3_dw_reduce<16>, dim3(rb), dim3(1024), 0, ctx->stream, part, slots, Cout, Cin, dw, acc,
-                           dbp, db);
-    else
-        hipLaunchKernelGGL(k_conv3_dw_reduce<4>, dim3(rb), dim3(256), 0, ctx->stream, part, slots, Cout, Cin, dw, acc,
-                           dbp, db);
+    reduce_dw(ctx, part, slots, Cout, Cin, dw, acc, dbp, db);
     *st = OM_LAUNCH_CHECK(ctx, "om_conv2d_bwd dw");
     return true;
 }
