@@ -11,7 +11,7 @@
 //
 // Operands the split does not carry take the fp32 instruction: an infinity or NaN (or a value that rounds past the
 // largest bf16) makes some partial product non-finite, and operands below about 2^-110, whose low part underflows,
-// leave sums below 2^-90. A wavefront whose finished sums show either recomputes its tile with
+// leave sums below 2^-90 (unless they meet operands above about 2^20: such terms keep the bits that bf16 still holds). A wavefront whose finished sums show either recomputes its tile with
 // v_mfma_f32_16x16x4_f32 straight from global memory, so such values come out as that instruction gives them.
 //
 // A workgroup is MG x KG wavefronts and computes BM x BN = (16 TM MG) x (16 TN) of C. Each wavefront owns 16 TM rows
