@@ -162,16 +162,16 @@ __global__ void __launch_bounds__(kThreads, 3) k_conv3_dw_s(Args a) {
             mma6(fg, f2, acc[2], low[2]);
         }
     }
-    unsigned big = 0, small = 0xFFFFFFFFu;
+    unsigned big = 0;
 #pragma unroll
     for (int t = 0; t < 3; t++) {
-        acc[t] += low[t];
+        finish_sums(acc[t], low[t]);
 #pragma unroll
-        for (int e = 0; e < 16; e++) note(acc[t][e], big, small);
+        for (int e = 0; e < 16; e++) note(acc[t][e], big);
     }
     // element e: output channel 8 (e / 4) + 4 hg + e % 4 of the wavefront's 32
     float *dst = a.part + (((int64_t)slot * a.cout + co0 + 32 * blk + 4 * hg) * 9 + 3 * ky) * a.cin + ci0 + l32;
-    if (beyond(big, small)) {  // values the split does not carry: this wavefront's sums in fp32 from global memory
+    if (beyond(big)) {  // values the split does not carry: this wavefront's sums in fp32 from global memory
 #pragma unroll 1
         for (int k = 0; k < 48; k++) {
             const int t = k % 3, e = k / 3, co = 8 * (e >> 2) + (e & 3);

@@ -162,16 +162,16 @@ __global__ void __launch_bounds__(64 * NW, 2) k_conv3_s(Args a) {
         }
         __syncthreads();
     }
-    unsigned big = 0, small = 0xFFFFFFFFu;
+    unsigned big = 0;
 #pragma unroll
     for (int i = 0; i < CB; i++) {
-        acc[i] += low[i];
+        finish_sums(acc[i], low[i]);
 #pragma unroll
-        for (int e = 0; e < 16; e++) note(acc[i][e], big, small);
+        for (int e = 0; e < 16; e++) note(acc[i][e], big);
     }
     const bool part = a.nsplit > 1;
     float *dst = (part ? a.ws + (int64_t)split * a.N * a.cout * P : a.out) + ((int64_t)n * a.cout + co0) * P + p;
-    if (beyond(big, small)) {  // values the split does not carry: this wavefront's outputs in fp32 from global memory
+    if (beyond(big)) {  // values the split does not carry: this wavefront's outputs in fp32 from global memory
         if (p >= P) return;
         const int oy = p / a.W, ox = p % a.W;
 #pragma unroll 1

@@ -9,10 +9,10 @@
 // operands) the relative error is 0.32-0.43 of the fp32 instruction's (K 384: 1.07e-7 against 3.5e-7; K 16384: 8.1e-7
 // against 2.3e-6).
 //
-// Operands the split does not carry take the fp32 instruction: an infinity or NaN (or a value that rounds past the
-// largest bf16) makes some partial product non-finite, and operands below about 2^-110, whose low part underflows,
-// leave sums below 2^-90 (unless they meet operands above about 2^20: such terms keep the bits that bf16 still holds). A wavefront whose finished sums show either recomputes its tile with
-// v_mfma_f32_16x16x4_f32 straight from global memory, so such values come out as that instruction gives them.
+// Operands are scaled by 2^24 on their way in, so no part of the smallest subnormal underflows, and the sums by 2^-48 on their
+// way out (om_split.hpp). What the scaled range does not hold takes the fp32 instruction: infinities, NaN, operands of 2^104
+// and sums of 2^80 leave a non-finite sum, and a wavefront that finds one among its finished sums recomputes its tile with
+// v_mfma_f32_32x32x2_f32 straight from global memory, so such values come out as that instruction gives them.
 //
 // A workgroup is MG x KG wavefronts and computes BM x BN = (16 TM MG) x (16 TN) of C. Each wavefront owns 16 TM rows
 // and all BN columns, so its A fragments are used by no other wavefront: it loads them from global memory straight
@@ -447,14 +447,14 @@ __device__ __forceinline__ void tile(const Params &p, int tm, int tn, int zz) {
         __syncthreads();
     }
 
-    unsigned big = 0, small = 0xFFFFFFFFu;
+    unsigned big = 0;
 #pragma unroll
     for (int j = 0; j < TN; j++) {
-        acc[j] += low[j];
+        finish_sums(acc[j], low[j]);
 #pragma unroll
-        for (int e = 0; e < 16; e++) note(acc[j][e], big, small);
+        for (int e = 0; e < 16; e++) note(acc[j][e], big);
     }
-    if (beyond(big, small)) {
+    if (beyond(big)) {
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             // column of the lane's LDS row, as the loads and the epilogue place it

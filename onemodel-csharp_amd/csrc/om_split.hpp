@@ -15,13 +15,21 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
 
-// Two fp32 values split into packed bf16 pairs, each part rounded to nearest. (v_dot2_f32_bf16 would give a residual in
-// one instruction, but it shares the matrix pipe: beside an MFMA it costs 16 cycles, the unpack and subtraction 8.)
+// Operands are scaled by 2^24 before they are split and finished sums scaled back by 2^-48, both exactly: the lowest part of
+// the smallest subnormal is then 2^-125, a normal bf16 value, so nothing of any operand below 2^104 is lost to bf16's range,
+// whatever it is multiplied with. Larger ones become infinite, as sums of 2^80 do, and are recomputed (beyond()). The price is
+// one multiplication beside the five and a half operations a value's split takes.
+constexpr float kScale = 0x1p24f, kUnscale = 0x1p-48f;
+
+// Two fp32 values, scaled, split into packed bf16 pairs, each part rounded to nearest. (v_dot2_f32_bf16 would give a residual
+// in one instruction, but it shares the matrix pipe: beside an MFMA it costs 16 cycles, the unpack and subtraction 8.)
 __device__ __forceinline__ uint32_t pack2(float x0, float x1) {
     const bf16x2 v = {(__bf16)x0, (__bf16)x1};
     return __builtin_bit_cast(uint32_t, v);
 }
 __device__ __forceinline__ void split2(float x0, float x1, uint32_t &h, uint32_t &m, uint32_t &l) {
+    x0 *= kScale;
+    x1 *= kScale;
     h = pack2(x0, x1);
     asm("" : "+v"(h));  // else the compiler converts x0 a second time instead of shifting h
     const float r0 = x0 - __uint_as_float(h << 16), r1 = x1 - __uint_as_float(h & 0xFFFF0000u);
@@ -61,15 +69,17 @@ __device__ __forceinline__ void mma6(const u32x4 (&a)[3], const u32x4 (&b)[3], f
     acc = mma(a[0], b[0], acc);
 }
 
-// Whether finished sums hold one that the split could not carry: non-finite, or so small (below 2^-90 and not zero) that
-// low parts may have underflowed. `big` and `small` collect over the sums of a lane (start at 0 and all ones).
-__device__ __forceinline__ void note(float v, unsigned &big, unsigned &small) {
+// A finished block of sums, scaled back.
+__device__ __forceinline__ void finish_sums(floatx16 &acc, const floatx16 &low) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = (acc[e] + low[e]) * kUnscale;
+}
+// Whether a wavefront's finished sums hold one that the split could not carry: an operand or a sum past the scaled range
+// leaves an infinity or a NaN. `big` collects over the sums of a lane (start at 0).
+__device__ __forceinline__ void note(float v, unsigned &big) {
     const unsigned u = __float_as_uint(v) & 0x7FFFFFFFu;
     big = u > big ? u : big;
-    small = u - 1u < small ? u - 1u : small;  // zero becomes the largest: exact zeros are fine
 }
-__device__ __forceinline__ bool beyond(unsigned big, unsigned small) {
-    return __any(big >= 0x7F800000u || small < 0x12800000u - 1u);
-}
+__device__ __forceinline__ bool beyond(unsigned big) { return __any(big >= 0x7F800000u); }
 
 }  // namespace oms

@@ -73,3 +73,20 @@ def test_values_the_split_does_not_carry(dev):
         assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
         assert np.all(np.abs(got[fin] - want[fin]) <= bound[fin])
         assert np.array_equal(dev.get(DB)[[5, 6]], np.float32([np.inf, np.inf]))
+
+
+# exponents of the tiny operand (the last two pairs: subnormals) and of its partner
+@pytest.mark.parametrize("et,ew", [(-115, 26), (-120, 40), (-125, 60), (-135, 100), (-145, 100), (-140, 0)])
+def test_tiny_operands_beside_large_ones(dev, et, ew):
+    """Operands down to the smallest subnormals times operands up to 2^100, whichever of the two is tiny: every term keeps all
+    its bits. The bound is test_edges's, and for sums that are subnormal themselves half a unit of the last place a term."""
+    N, Cin, Cout, H, W = 40, 32, 64, 9, 13
+    rng = np.random.default_rng(23)
+    x0, g0 = (rng.standard_normal((N, c, H, W)).astype(np.float32) for c in (Cin, Cout))
+    for ex, eg in ((et, ew), (ew, et)):
+        x, g = np.ldexp(x0, ex), np.ldexp(g0, eg)
+        DW = dev.empty((Cout, Cin, 3, 3))
+        dev.call("om_conv2d_bwd", dev.put(g), dev.put(x), dev.put(np.zeros(DW.shape, np.float32)), None, DW, None, N, Cin, H,
+                 W, Cout, 3, 3, 1, 1, 0, 0)
+        bound = N * H * W * (2.0 ** -24 * dw64(np.abs(g), np.abs(x)) + 2.0 ** -150)
+        assert np.all(np.abs(dev.get(DW) - dw64(g, x)) <= bound), (ex, eg)

@@ -5,6 +5,8 @@ operands the three-way bf16 split does not carry, against float64 over the zero-
 Tolerance: the sequential-accumulation bound k 2^-24 sum |w||x| over the k = 9 Cin terms (the kernel's own rounding count
 is lower: one per 16 terms and six per 16 on sums 2^-8 as large), and a rounding of each later addition.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -86,3 +88,49 @@ def test_values_the_split_does_not_carry(dev, N, C, H, W):
             assert np.array_equal(np.isnan(got), np.isnan(want))
             assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
             assert np.all(np.abs(got[fin] - want[fin]) <= bound[fin])
+
+
+@pytest.mark.parametrize("N,C,H,W", [(16, 32, 17, 19), (8, 64, 6, 9)])
+@pytest.mark.parametrize("tiny_w", [False, True])
+def test_tiny_operands_beside_large_ones(dev, N, C, H, W, tiny_w):
+    """Images (or filters) down to the smallest subnormals times filters (images) up to 2^100: every term keeps all its bits.
+    The bound is test_edges's, and for sums that are subnormal themselves half a unit of the last place a term."""
+    rng = np.random.default_rng(19)
+    tiny = np.ldexp(1.0, [-112, -118, -124, -127, -133, -137, -142, -147])
+    wide = np.ldexp(1.0, [0, 10, 20, 40, 60, 100])
+    si, sf = (wide, tiny) if tiny_w else (tiny, wide)
+    x = (rng.standard_normal((N, C, H, W)) * np.resize(si, N)[:, None, None, None]).astype(np.float32)
+    w0 = rng.standard_normal((C, C, 3, 3))
+    X, Y, B = dev.put(x), dev.empty(x.shape), dev.put(np.zeros(C, np.float32))
+    for flip in (False, True):
+        w = (w0 * (np.resize(sf, C)[None, :, None, None] if flip else np.resize(sf, C)[:, None, None, None])).astype(np.float32)
+        if flip:
+            dev.call("om_conv2d_bwd", X, X, dev.put(w), Y, dev.empty(w.shape), dev.empty((C,)), N, C, H, W, C, 3, 3, 1, 1, 0, 0)
+        else:
+            dev.call("om_conv2d_fwd", X, dev.put(w), B, Y, N, C, H, W, C, 3, 3, 1, 1)
+        wf = turned(w) if flip else w
+        bound = 9 * C * (2.0 ** -24 * conv64(np.abs(x), np.abs(wf)) + 2.0 ** -150)
+        assert np.all(np.abs(dev.get(Y) - conv64(x, wf)) <= bound)
+
+
+def test_tiny_sums_cost_no_more(dev):
+    """Gradients of confidently classified samples are around e^-65: nothing of a convolution over them is slower. (Sums below
+    2^-90 once took a path a hundred times as long; the factor 2 is for the clock's noise.)"""
+    N, C, H, W = 16, 64, 28, 28
+    rng = np.random.default_rng(3)
+    w, dx, dw, db = dev.put(rng.standard_normal((C, C, 3, 3)).astype(np.float32)), dev.empty((N, C, H, W)), dev.empty((C, C, 3, 3)), dev.empty((C,))
+    x = dev.put(rng.standard_normal((N, C, H, W)).astype(np.float32))
+    best = []
+    for scale in (1.0, 2.0 ** -94):
+        g = dev.put((rng.standard_normal((N, C, H, W)) * scale).astype(np.float32))
+        args = (g, x, w, dx, dw, db, N, C, H, W, C, 3, 3, 1, 1, 0, 0)
+        times = []
+        for _ in range(6):
+            dev.get(db)
+            t = time.perf_counter()
+            for _ in range(10):
+                dev.call("om_conv2d_bwd", *args)
+            dev.get(db)
+            times.append(time.perf_counter() - t)
+        best.append(min(times))
+    assert best[1] <= 2 * best[0]

@@ -111,3 +111,22 @@ def test_grouped_weight_gradients(dev, rows, sizes):
         assert np.all(np.abs(dev.get(b[2]) - g.T @ x) <= rows * 2.0 ** -24 * (np.abs(g).T @ np.abs(x)))
         s = g.sum(0)
         assert np.all(np.abs(dev.get(b[3]) - s) <= 2.0 ** -23 * np.abs(s) + 1e-12 * np.abs(g).sum(0))  # summed in double
+
+
+# exponents of the tiny operand (the last two pairs: subnormals) and of its partner
+TINY_WIDE = [(-115, 26), (-120, 40), (-125, 60), (-135, 100), (-145, 100), (-140, 0)]
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(130, 71, 203), (512, 384, 384)])
+def test_tiny_operands_beside_large_ones(dev, ta, tb, m, n, k):
+    """Operands down to the smallest subnormals times operands up to 2^100, whichever of the two is tiny: every term keeps all
+    its bits. The bound is test_edges's, and for sums that are subnormal themselves half a unit of the last place a term."""
+    rng = np.random.default_rng(17)
+    A0, B0, _, _ = operands(rng, ta, tb, m, n, k)
+    for pair in TINY_WIDE:
+        for ea, eb in (pair, pair[::-1]):
+            A, B = np.ldexp(A0, ea), np.ldexp(B0, eb)
+            A64, B64 = (A.T if ta else A).astype(np.float64), (B.T if tb else B).astype(np.float64)
+            bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + k * 2.0 ** -150
+            assert np.all(np.abs(product(dev, ta, tb, A, B, m, n, k) - A64 @ B64) <= bound), (ea, eb)
