@@ -171,33 +171,45 @@ __global__ void __launch_bounds__(kThreads, 3) k_conv3_dw_s(Args a) {
     }
     // element e: output channel 8 (e / 4) + 4 hg + e % 4 of the wavefront's 32
     float *dst = a.part + (((int64_t)slot * a.cout + co0 + 32 * blk + 4 * hg) * 9 + 3 * ky) * a.cin + ci0 + l32;
-    if (beyond(big)) {  // values the split does not carry: this wavefront's sums in fp32 from global memory
-#pragma unroll 1
-        for (int k = 0; k < 48; k++) {
-            const int t = k % 3, e = k / 3, co = 8 * (e >> 2) + (e & 3);
-            float v = 0.0f;
-#pragma unroll 1
-            for (int item = i0; item < i1; item++) {
-                const int seg = item % a.segs, band = item / a.segs % a.bands, n = item / a.segs / a.bands;
-                const float *gg = a.g + ((int64_t)n * a.cout + co0 + 32 * blk + 4 * hg + co) * P;
-                const float *xx = a.x + ((int64_t)n * a.cin + ci0 + l32) * P;
-#pragma unroll 1
-                for (int oy = band * a.RB; oy < min(a.H, (band + 1) * a.RB); oy++)
-#pragma unroll 1
-                    for (int ox = seg * a.SG * 8; ox < min(a.W, (seg + 1) * a.SG * 8); ox++) {
-                        const int iy = oy + ky - 1, ix = ox + t - 1;
-                        const bool in = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-                        v = fmaf(gg[oy * a.W + ox], in ? xx[iy * a.W + ix] : 0.0f, v);
-                    }
-            }
-            dst[((int64_t)co * 9 + t) * a.cin] = v;
-        }
-    } else {
+    if (beyond(big)) {  // values the split does not carry: this wavefront's sums on the fp32 instruction, from global memory
 #pragma unroll
         for (int t = 0; t < 3; t++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) dst[((int64_t)(8 * (e >> 2) + (e & 3)) * 9 + t) * a.cin] = acc[t][e];
+            for (int e = 0; e < 16; e++) acc[t][e] = 0.0f;
+#pragma unroll 1
+        for (int item = i0; item < i1; item++) {
+            const int seg = item % a.segs, band = item / a.segs % a.bands, n = item / a.segs / a.bands;
+            const float *gg = a.g + ((int64_t)n * a.cout + co0 + 32 * blk + l32) * P;
+            const float *xx = a.x + ((int64_t)n * a.cin + ci0 + l32) * P;
+            const int ox1 = min(a.W, (seg + 1) * a.SG * 8);
+#pragma unroll 1
+            for (int oy = band * a.RB; oy < min(a.H, (band + 1) * a.RB); oy++) {
+                const int iy = oy + ky - 1;
+                const bool row = (unsigned)iy < (unsigned)a.H;
+                const float *gr = gg + oy * a.W, *xr = xx + (row ? iy : oy) * a.W;
+#pragma unroll 1
+                for (int ox = seg * a.SG * 8; ox < ox1; ox += 8) {
+#pragma unroll
+                    for (int j = 0; j < 8; j += 2) {
+                        const int px = ox + j + hg;
+                        const bool has = px < ox1;
+                        const float gv = gr[min(px, a.W - 1)];
+#pragma unroll
+                        for (int t = 0; t < 3; t++) {
+                            const int ix = px + t - 1;
+                            const float v = xr[min(max(ix, 0), a.W - 1)];
+                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                has ? gv : 0.0f, has && row && (unsigned)ix < (unsigned)a.W ? v : 0.0f, acc[t], 0, 0, 0);
+                        }
+                    }
+                }
+            }
+        }
     }
+#pragma unroll
+    for (int t = 0; t < 3; t++)
+#pragma unroll
+        for (int e = 0; e < 16; e++) dst[((int64_t)(8 * (e >> 2) + (e & 3)) * 9 + t) * a.cin] = acc[t][e];
     if (!do_db) return;  // uniform over the workgroup
     __syncthreads();
     double *ds = reinterpret_cast<double *>(sh);

@@ -169,35 +169,31 @@ __global__ void __launch_bounds__(64 * NW, 2) k_conv3_s(Args a) {
 #pragma unroll
         for (int e = 0; e < 16; e++) note(acc[i][e], big);
     }
+    if (beyond(big)) {  // values the split does not carry: this wavefront's sums on the fp32 instruction, from global memory
+        const int pc = min(p, P - 1), oy = pc / a.W, ox = pc % a.W;
+#pragma unroll
+        for (int i = 0; i < CB; i++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[i][e] = 0.0f;
+#pragma unroll 1
+        for (int c0 = c_beg; c0 < c_end; c0 += 2) {
+            const int c = c0 + g;
+            const float *x = inn + (int64_t)c * P;
+            const float *ww = a.wt + (FLIP ? (int64_t)c * a.cout + co0 + l32 : (int64_t)(co0 + l32) * a.cin + c) * 9;
+#pragma unroll
+            for (int t = 0; t < 9; t++) {
+                const int iy = oy + t / 3 - 1, ix = ox + t % 3 - 1;
+                const bool in = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
+                const float v = x[in ? iy * a.W + ix : 0];
+#pragma unroll
+                for (int i = 0; i < CB; i++)  // an infinite weight on the border: NaN
+                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(ww[(int64_t)32 * 9 * i * (FLIP ? 1 : a.cin) + (FLIP ? 8 - t : t)],
+                                                                  in ? v : 0.0f, acc[i], 0, 0, 0);
+            }
+        }
+    }
     const bool part = a.nsplit > 1;
     float *dst = (part ? a.ws + (int64_t)split * a.N * a.cout * P : a.out) + ((int64_t)n * a.cout + co0) * P + p;
-    if (beyond(big)) {  // values the split does not carry: this wavefront's outputs in fp32 from global memory
-        if (p >= P) return;
-        const int oy = p / a.W, ox = p % a.W;
-#pragma unroll 1
-        for (int co = g; co < BM; co += 2) {
-            float v = 0.0f;
-#pragma unroll 1
-            for (int c = c_beg; c < c_end; c++) {
-                const float *x = inn + (int64_t)c * P;
-                const float *ww = a.wt + (FLIP ? (int64_t)c * a.cout + co0 + co : (int64_t)(co0 + co) * a.cin + c) * 9;
-#pragma unroll 1
-                for (int t = 0; t < 9; t++) {
-                    const int iy = oy + t / 3 - 1, ix = ox + t % 3 - 1;
-                    const bool in = (unsigned)iy < (unsigned)a.H && (unsigned)ix < (unsigned)a.W;
-                    v = fmaf(ww[FLIP ? 8 - t : t], in ? x[iy * a.W + ix] : 0.0f, v);  // an infinite weight on the border: NaN
-                }
-            }
-            float *d = dst + (int64_t)co * P;
-            if (!part) {
-                if (a.bias) v = v + a.bias[co0 + co];
-                if (a.relu) v = relu1(v);
-                if (a.acc) v = *d + v;
-            }
-            *d = v;
-        }
-        return;
-    }
     // element e of block i: channel 32 i + 8 (e / 4) + 4 g + e % 4. Each pass runs over all of them before the next, so that
     // its loads or stores are in flight together.
     auto each = [&](auto f) {

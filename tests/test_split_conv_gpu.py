@@ -113,24 +113,26 @@ def test_tiny_operands_beside_large_ones(dev, N, C, H, W, tiny_w):
         assert np.all(np.abs(dev.get(Y) - conv64(x, wf)) <= bound)
 
 
-def test_tiny_sums_cost_no_more(dev):
-    """Gradients of confidently classified samples are around e^-65: nothing of a convolution over them is slower. (Sums below
-    2^-90 once took a path a hundred times as long; the factor 2 is for the clock's noise.)"""
+@pytest.mark.parametrize("scale,factor", [(2.0 ** -94, 2), (np.nan, 8)])
+def test_no_values_take_a_slow_path(dev, scale, factor):
+    """Gradients of confidently classified samples are around e^-65 and cost what others do (the factor 2 is for the clock's
+    noise); those of a diverged step run on the fp32 instruction, 2.4 times as long. (Loops over single terms once took 12 and
+    30 times as long.)"""
     N, C, H, W = 16, 64, 28, 28
     rng = np.random.default_rng(3)
-    w, dx, dw, db = dev.put(rng.standard_normal((C, C, 3, 3)).astype(np.float32)), dev.empty((N, C, H, W)), dev.empty((C, C, 3, 3)), dev.empty((C,))
-    x = dev.put(rng.standard_normal((N, C, H, W)).astype(np.float32))
+    x, g = (rng.standard_normal((N, C, H, W)).astype(np.float32) for _ in range(2))
+    X, Wt, DX = dev.put(x), dev.put(rng.standard_normal((C, C, 3, 3)).astype(np.float32)), dev.empty(x.shape)
+    DW, DB = dev.empty((C, C, 3, 3)), dev.empty((C,))
     best = []
-    for scale in (1.0, 2.0 ** -94):
-        g = dev.put((rng.standard_normal((N, C, H, W)) * scale).astype(np.float32))
-        args = (g, x, w, dx, dw, db, N, C, H, W, C, 3, 3, 1, 1, 0, 0)
+    for s in (1.0, scale):
+        G = dev.put(g * np.float32(s))
         times = []
         for _ in range(6):
-            dev.get(db)
+            dev.get(DB)
             t = time.perf_counter()
             for _ in range(10):
-                dev.call("om_conv2d_bwd", *args)
-            dev.get(db)
+                dev.call("om_conv2d_bwd", G, X, Wt, DX, DW, DB, N, C, H, W, C, 3, 3, 1, 1, 0, 0)
+            dev.get(DB)
             times.append(time.perf_counter() - t)
         best.append(min(times))
-    assert best[1] <= 2 * best[0]
+    assert best[1] <= factor * best[0]
