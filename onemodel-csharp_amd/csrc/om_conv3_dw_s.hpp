@@ -172,10 +172,11 @@ __global__ void __launch_bounds__(kThreads, 3) k_conv3_dw_s(Args a) {
     // element e: output channel 8 (e / 4) + 4 hg + e % 4 of the wavefront's 32
     float *dst = a.part + (((int64_t)slot * a.cout + co0 + 32 * blk + 4 * hg) * 9 + 3 * ky) * a.cin + ci0 + l32;
     if (beyond(big)) {  // values the split does not carry: this wavefront's sums on the fp32 instruction, from global memory
+        floatx16 s[3];
 #pragma unroll
         for (int t = 0; t < 3; t++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[t][e] = 0.0f;
+            for (int e = 0; e < 16; e++) s[t][e] = 0.0f;
 #pragma unroll 1
         for (int item = i0; item < i1; item++) {
             const int seg = item % a.segs, band = item / a.segs % a.bands, n = item / a.segs / a.bands;
@@ -198,13 +199,15 @@ __global__ void __launch_bounds__(kThreads, 3) k_conv3_dw_s(Args a) {
                         for (int t = 0; t < 3; t++) {
                             const int ix = px + t - 1;
                             const float v = xr[min(max(ix, 0), a.W - 1)];
-                            acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                                has ? gv : 0.0f, has && row && (unsigned)ix < (unsigned)a.W ? v : 0.0f, acc[t], 0, 0, 0);
+                            s[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                                has ? gv : 0.0f, has && row && (unsigned)ix < (unsigned)a.W ? v : 0.0f, s[t], 0, 0, 0);
                         }
                     }
                 }
             }
         }
+#pragma unroll
+        for (int t = 0; t < 3; t++) take_beyond(acc[t], s[t]);
     }
 #pragma unroll
     for (int t = 0; t < 3; t++)

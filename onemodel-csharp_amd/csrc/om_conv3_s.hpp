@@ -170,11 +170,12 @@ __global__ void __launch_bounds__(64 * NW, 2) k_conv3_s(Args a) {
         for (int e = 0; e < 16; e++) note(acc[i][e], big);
     }
     if (beyond(big)) {  // values the split does not carry: this wavefront's sums on the fp32 instruction, from global memory
+        floatx16 f[CB];
         const int pc = min(p, P - 1), oy = pc / a.W, ox = pc % a.W;
 #pragma unroll
         for (int i = 0; i < CB; i++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[i][e] = 0.0f;
+            for (int e = 0; e < 16; e++) f[i][e] = 0.0f;
 #pragma unroll 1
         for (int c0 = c_beg; c0 < c_end; c0 += 2) {
             const int c = c0 + g;
@@ -187,10 +188,12 @@ __global__ void __launch_bounds__(64 * NW, 2) k_conv3_s(Args a) {
                 const float v = x[in ? iy * a.W + ix : 0];
 #pragma unroll
                 for (int i = 0; i < CB; i++)  // an infinite weight on the border: NaN
-                    acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(ww[(int64_t)32 * 9 * i * (FLIP ? 1 : a.cin) + (FLIP ? 8 - t : t)],
-                                                                  in ? v : 0.0f, acc[i], 0, 0, 0);
+                    f[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(ww[(int64_t)32 * 9 * i * (FLIP ? 1 : a.cin) + (FLIP ? 8 - t : t)],
+                                                                  in ? v : 0.0f, f[i], 0, 0, 0);
             }
         }
+#pragma unroll
+        for (int i = 0; i < CB; i++) take_beyond(acc[i], f[i]);
     }
     const bool part = a.nsplit > 1;
     float *dst = (part ? a.ws + (int64_t)split * a.N * a.cout * P : a.out) + ((int64_t)n * a.cout + co0) * P + p;

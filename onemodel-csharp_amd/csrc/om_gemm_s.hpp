@@ -461,14 +461,15 @@ __device__ __forceinline__ void tile(const Params &p, int tm, int tn, int zz) {
             const int col = 32 * j + l32;
             const int cc = BK_ ? min(col, p.n - 1 - n0) : LB::shifted(col / LB::RV * LB::RV, p.n - n0) + col % LB::RV;
             const float *b = B + (BK_ ? (int64_t)(n0 + cc) * p.ldb : (int64_t)(n0 + cc));
+            floatx16 t;
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[j][e] = 0.0f;
+            for (int e = 0; e < 16; e++) t[e] = 0.0f;
 #pragma unroll 1
             for (int it = 0; it <= nit; it++) {  // the group's steps, then (group 0) the tail
                 const bool tail = it == nit;
                 const int k0 = tail ? kbeg + 32 * full : kat(it);
                 if (tail ? kg != 0 || k0 >= kend : k0 >= kbeg + 32 * full) continue;
-#pragma unroll
+#pragma unroll 1
                 for (int w = 0; w < 4; w++) {
                     float xa[4];
                     la.quad_tail(xa, w, k0, kend);
@@ -476,10 +477,11 @@ __device__ __forceinline__ void tile(const Params &p, int tm, int tn, int zz) {
                     for (int e = 0; e < 4; e++) {
                         const int k = k0 + 8 * w + 4 * g + e, kc = kclamp(k, kend);
                         const float v = BK_ ? b[kc] : b[(int64_t)kc * p.ldb];
-                        acc[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(k < kend ? v : 0.0f, xa[e], acc[j], 0, 0, 0);
+                        t = __builtin_amdgcn_mfma_f32_32x32x2f32(k < kend ? v : 0.0f, xa[e], t, 0, 0, 0);
                     }
                 }
             }
+            take_beyond(acc[j], t);
         }
     }
 

@@ -81,5 +81,10 @@ __device__ __forceinline__ void note(float v, unsigned &big) {
     big = u > big ? u : big;
 }
 __device__ __forceinline__ bool beyond(unsigned big) { return __any(big >= 0x7F800000u); }
+// Takes those sums, and only those, from `fp32`: a result depends on its own operands, not on what shares its wavefront.
+__device__ __forceinline__ void take_beyond(floatx16 &acc, const floatx16 &fp32) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[e] = (__float_as_uint(acc[e]) & 0x7FFFFFFFu) >= 0x7F800000u ? fp32[e] : acc[e];
+}
 
 }  // namespace oms

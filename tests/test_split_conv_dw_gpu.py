@@ -90,3 +90,18 @@ def test_tiny_operands_beside_large_ones(dev, et, ew):
                  W, Cout, 3, 3, 1, 1, 0, 0)
         bound = N * H * W * (2.0 ** -24 * dw64(np.abs(g), np.abs(x)) + 2.0 ** -150)
         assert np.all(np.abs(dev.get(DW) - dw64(g, x)) <= bound), (ex, eg)
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 2.0 ** 105])
+def test_a_channel_does_not_depend_on_its_neighbours(dev, bad):
+    """A value the split does not carry changes its own channels' gradients and no bit of another."""
+    N, Cin, Cout, H, W = 40, 32, 64, 9, 13
+    rng = np.random.default_rng(37)
+    x, g = (rng.standard_normal((N, c, H, W)).astype(np.float32) for c in (Cin, Cout))
+    zero, out = np.zeros((Cout, Cin, 3, 3), np.float32), []
+    for v, u in ((x[2, 3, 5, 9], g[1, 40, 0, 0]), (bad, bad)):
+        x[2, 3, 5, 9], g[1, 40, 0, 0] = v, u
+        DW = dev.empty(zero.shape)
+        dev.call("om_conv2d_bwd", dev.put(g), dev.put(x), dev.put(zero), None, DW, None, N, Cin, H, W, Cout, 3, 3, 1, 1, 0, 0)
+        out.append(np.delete(np.delete(dev.get(DW), 3, 1), 40, 0))
+    assert np.array_equal(out[0], out[1])

@@ -136,3 +136,24 @@ def test_no_values_take_a_slow_path(dev, scale, factor):
             times.append(time.perf_counter() - t)
         best.append(min(times))
     assert best[1] <= factor * best[0]
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 2.0 ** 105])
+def test_a_pixel_does_not_depend_on_its_neighbours(dev, bad):
+    """A value the split does not carry changes the sums that it is part of and no bit of another."""
+    N, C, H, W = 6, 32, 17, 19
+    rng = np.random.default_rng(31)
+    x = rng.standard_normal((N, C, H, W)).astype(np.float32)
+    w = dev.put(rng.standard_normal((C, C, 3, 3)).astype(np.float32))
+    b, y = dev.put(np.zeros(C, np.float32)), dev.empty(x.shape)
+    keep = np.ones(x.shape, bool)
+    keep[2, :, 4:7, 8:11] = False
+    out = []
+    for v in (x[2, 3, 5, 9], bad):
+        x[2, 3, 5, 9] = v
+        X = dev.put(x)
+        dev.call("om_conv2d_fwd", X, w, b, y, N, C, H, W, C, 3, 3, 1, 1)
+        out.append(dev.get(y)[keep])
+        dev.call("om_conv2d_bwd", X, X, w, y, dev.empty((C, C, 3, 3)), None, N, C, H, W, C, 3, 3, 1, 1, 0, 0)
+        out.append(dev.get(y)[keep])
+    assert np.array_equal(out[0], out[2]) and np.array_equal(out[1], out[3])

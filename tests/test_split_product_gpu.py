@@ -130,3 +130,18 @@ def test_tiny_operands_beside_large_ones(dev, ta, tb, m, n, k):
             A64, B64 = (A.T if ta else A).astype(np.float64), (B.T if tb else B).astype(np.float64)
             bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + k * 2.0 ** -150
             assert np.all(np.abs(product(dev, ta, tb, A, B, m, n, k) - A64 @ B64) <= bound), (ea, eb)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(130, 71, 203), (512, 384, 384)])
+@pytest.mark.parametrize("bad", [np.inf, np.nan, 2.0 ** 105])
+def test_a_row_does_not_depend_on_its_neighbours(dev, ta, tb, m, n, k, bad):
+    """A value the split does not carry changes its own row (column) of the product and no bit of another."""
+    A, B, _, _ = operands(np.random.default_rng(29), ta, tb, m, n, k)
+    clean = product(dev, ta, tb, A, B, m, n, k)
+    A[(7, 37) if ta else (37, 7)] = bad
+    B[(20, 9) if tb else (9, 20)] = bad
+    got = product(dev, ta, tb, A, B, m, n, k)
+    keep = np.ones((m, n), bool)
+    keep[37], keep[:, 20] = False, False
+    assert np.array_equal(got[keep], clean[keep])
