@@ -297,21 +297,29 @@ Choice choose(int m, int n, int k, int batch, int cus) {
     return c;
 }
 
-// Short sums over few tiles on the tile-exact fp32 kernels: whole 64 x 96 (or 64 x 64) tiles, at most one per CU, and at
-// most five chunks of 32 k. Against the split-operand kernel (us, both ways timed back to back): 4096 x 384 at k 32 / 64
-// / 128 / 192 / 256 5.0 / 5.8 / 7.3 / 8.8 / 10.4 here and 6.1 / 7.6 / 8.7 / 9.6 / 10.3 there, 1024 x 256 4.2 / 4.4 / 5.5 /
-// 6.6 / 7.7 and 5.1 / 5.1 / 6.5 / 6.8 / 7.8; with more than a tile per CU the split kernel wins from k = 32 on (4096 x
-// 1536 11.1 and 10.6). Both operands K-contiguous take the chunks straight into LDS. Returns the tile width (0: the
-// product is not taken). A GELU epilogue's family is compiled in (0 none, 1 the reference's polynomials, 2 the pair of
-// stated error with the slope product).
+// Short sums over few tiles on the tile-exact fp32 kernels: whole 64 x 64 tiles, or 64 x 96 where those would be more than the
+// CUs, at most one per CU. A chunk of 32 k costs them 0.55 and 0.75 us, the split-operand kernel less but a longer start, so
+// the line lies at 288 (both operands K-contiguous, whose chunks go straight into LDS: 320), and lower where that kernel has
+// CUs left for k groups and splits, or whole rounds of four k groups (k = 256). Against it (us, k 160 / 224 / 288 / 320 / 384,
+// operands K-contiguous): 4096 x 384 8.7 / 9.6 / 11.2 / 12.2 / 13.7 here and 9.1 / 10.8 / 12.6 / 12.9 / 13.1 there, 1024 x 256 6.1
+// / 7.2 / 8.3 / 8.9 / 10.0 and 8.2 / 8.4 / 10.0 / 9.8 / 10.7, 64 x 64 5.7 / 6.8 / 7.9 / 8.5 / 9.5 and 7.9 / 8.0 / 8.2 / 7.8 /
+// 8.0; weight gradients of 1024 x 256 at k 256 / 288 / 320 8.7 / 9.3 / 10.0 and 8.3 / 10.7 / 10.1. With more than a tile per CU
+// the split kernel wins from k = 32 on (4096 x 1536 11.1 and 10.6). Returns the tile width (0: the product is not taken). A
+// GELU epilogue's family is compiled in (0 none, 1 the reference's polynomials, 2 the pair of stated error with the slope
+// product).
 static int short_tile(const Params &p, bool ta, bool tb, int batch, int cus) {
     const bool al = ((uintptr_t)p.a % 16 == 0) && ((uintptr_t)p.b % 16 == 0) && p.lda % 4 == 0 && p.ldb % 4 == 0 &&
                     p.sa_outer % 4 == 0 && p.sa_inner % 4 == 0 && p.sb_outer % 4 == 0 && p.sb_inner % 4 == 0;
-    if (!al || (ta && tb) || p.k <= 0 || p.k > 160 || p.k % 32 || p.m % 64) return 0;
-    const int bn = p.n % 96 == 0 ? 96 : p.n % 64 == 0 ? 64 : 0;
-    if (!bn || (int64_t)(p.m / 64) * (p.n / bn) * batch > cus) return 0;
+    if (!al || (ta && tb) || p.k <= 0 || p.k % 32 || p.m % 64) return 0;
     const int64_t ld = p.lda > p.ldb ? p.lda : p.ldb;
-    return ld * 96 < (int64_t)1 << 31 ? bn : 0;
+    if (ld * 96 >= (int64_t)1 << 31) return 0;
+    for (const int bn : {64, 96}) {
+        const int64_t tiles = (int64_t)(p.m / 64) * (p.n / bn) * batch;
+        if (p.n % bn || tiles > cus) continue;
+        const int most = bn == 96 && tiles * 2 <= cus ? 160 : !tb || tiles * 8 < cus ? 288 : 320;
+        return p.k <= most && (tb || p.k != 256) ? bn : 0;
+    }
+    return 0;
 }
 template <int BN>
 static void launch_short(const Params &p, bool ta, bool tb, int batch, hipStream_t st) {

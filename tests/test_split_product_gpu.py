@@ -145,3 +145,17 @@ def test_a_row_does_not_depend_on_its_neighbours(dev, ta, tb, m, n, k, bad):
     keep = np.ones((m, n), bool)
     keep[37], keep[:, 20] = False, False
     assert np.array_equal(got[keep], clean[keep])
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(64, 64, 192), (64, 64, 288), (64, 64, 320), (512, 384, 224), (1024, 256, 256), (1024, 256, 320),
+                                   (1024, 256, 352), (4096, 384, 288), (4096, 384, 320), (4096, 384, 352), (1024, 96, 160), (1024, 96, 192)])
+def test_short_sums_on_both_sides_of_the_rule(dev, ta, tb, m, n, k):
+    """Whole tiles with sums around the length up to which the fp32 kernels run, with bias and accumulation."""
+    rng = np.random.default_rng(m + k)
+    A, B, A64, B64 = operands(rng, ta, tb, m, n, k)
+    bias, c0 = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    got = product(dev, ta, tb, A, B, m, n, k, c0=c0.copy(), bias=bias, acc=1)
+    want = A64 @ B64 + bias + c0
+    bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + 2.0 ** -22 * (np.abs(bias) + np.abs(c0) + np.abs(want))
+    assert np.all(np.abs(got - want) <= bound)
