@@ -222,14 +222,17 @@ const int kSplits[] = {1, 2, 3, 4, 5, 6, 7, 8, 12, 16};
 
 // Estimated time (units of 0.08 us) of products of `tiles` workgroups in all, each `steps` 32-k steps long: every CU's
 // share of tiles, a fixed cost of each round of workgroups (first loads, epilogue; about 3 us), and with a split the
-// reduce (a launch, then the partial sums it reads at about 5 TB/s).
+// reduce: a launch of 3 us, the partial sums it reads at about 3 TB/s (they come from other XCDs), and where a row is not
+// whole quads its walk over the splits. (Priced at 2 us and 5 TB/s, products of few tiles split too often: 512 x 384 x 768 12.9
+// us in six splits, 10.9 in two; 768 x 768 x 1024 nn 21.8 and 15.8; 2 x 37 x 256 10.4 in four, 7.7 unsplit. Over 220 shapes the
+// choice was 4.5 % above the best on average, now 2.2 %.)
 double s_time(const SConfig &c, int64_t tiles, int steps, int cus) {
     const int64_t share = (tiles + cus - 1) / cus, rounds = (tiles + (int64_t)cus * c.per_cu - 1) / ((int64_t)cus * c.per_cu);
     const int blocks = c.bm * c.bn / 1024, st = (steps + c.kg - 1) / c.kg * c.kg;
     return (double)share * blocks * (st * (share > 1 ? c.cost : c.alone) + 1.5) + 38.0 * (double)rounds;
 }
-double reduce_time(int splits, double outputs) {
-    return splits > 1 ? 25.0 + (splits + 1.0) * outputs * 4.0 / 5.0e6 / 0.08 : 0.0;
+double reduce_time(int splits, double outputs, bool ragged) {
+    return splits > 1 ? 40.0 + (splits + 1.0) * outputs * 4.0 / 3.0e6 / 0.08 + (ragged ? 4.0 * splits : 0.0) : 0.0;
 }
 struct SChoice {
     const SConfig *c;
@@ -244,8 +247,9 @@ SChoice choose_s(int count, const int *m, const int *n, int k, int batch, int cu
     for (int i = 0; i < count; i++) outputs += (double)m[i] * n[i];
     for (const SConfig &c : kS) {
         int64_t tiles = 0;
-        bool whole = true;
+        bool whole = true, ragged = false;
         for (int i = 0; i < count; i++) {
+            ragged = ragged || n[i] % 4;
             tiles += (int64_t)((m[i] + c.bm - 1) / c.bm) * ((n[i] + c.bn - 1) / c.bn) * batch;
             whole = whole && m[i] % c.bm == 0 && n[i] % c.bn == 0;
         }
@@ -254,7 +258,7 @@ SChoice choose_s(int count, const int *m, const int *n, int k, int batch, int cu
             const int len = sp > 1 ? split_len(k, sp, 32 * c.kg) : k;
             if (sp > 1 && (int64_t)(sp - 1) * len >= k) continue;
             const bool exact = whole && k % (32 * c.kg) == 0;
-            const double t = (s_time(c, tiles * sp, (len + 31) / 32, cus) * (exact ? 1.0 : 1.08)) + reduce_time(sp, outputs);
+            const double t = (s_time(c, tiles * sp, (len + 31) / 32, cus) * (exact ? 1.0 : 1.08)) + reduce_time(sp, outputs, ragged);
             if (t < best_t) {
                 best_t = t;
                 best = SChoice{&c, sp, len, exact};
