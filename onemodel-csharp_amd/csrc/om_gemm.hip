@@ -3,7 +3,7 @@
 // A product runs the split-operand kernel (om_gemm_s.hpp) on a tile and a K split that depend on the shape and the CU
 // count only (choose_s); short sums over few whole tiles run the tile-exact fp32 kernels (om_gemm_x.hpp, short_tile);
 // what neither takes (both operands transposed, fewer than four columns, sums of fewer than 16 terms, leading dimensions
-// past 32-bit byte offsets) the guarded fp32 kernel k_gemm.
+// past 32-bit byte offsets) and a few small products (general_wins) the guarded fp32 kernel k_gemm.
 #include <cstdlib>
 #include <cstring>
 #include <utility>
@@ -274,15 +274,30 @@ bool s_takes(const Params &p, bool ta, bool tb) {
     const int64_t ld = p.lda > p.ldb ? p.lda : p.ldb;
     return !(ta && tb) && p.n >= 4 && p.k >= 16 && p.k < INT32_MAX - 4096 && ld < ((int64_t)1 << 22);
 }
+// Products that the split-operand kernel could take and the guarded fp32 kernel is faster at (us there and here, the range over
+// the three layouts):
+//   at most 32 x 32 outputs (of batches 16 x 16) with less than two steps of 32 k: 16 x 16 x 16 5.6-6.3 and 5.0-5.7, 31 x 32 x 40
+//   7.2-8.4 and 6.5-6.9;
+//   a few tiles with 64 < k < 352 ragged, which that kernel splits into slices of at least 32 k: 100 x 100 x 163 / 333 9.6-10.6 /
+//   11.1-12.1 and 8.6-8.8 / 8.6-8.9 (k 390: 8.4-10.2 and 11.3-11.7; rows that are not whole quads, whose reduce is slow, no worse
+//   here);
+//   16 terms, half a step, over many outputs: 13685 x 1474 37.9-44.7 and 34.4-35.2 (1517 x 391 6.8-7.5 and 8.8-9.1).
+// Bias gradients and MSE terms ride along with the split-operand kernel only, so products that carry them stay there.
+bool general_wins(const Params &p, int batch) {
+    if (p.db || p.mse_t) return false;
+    const int64_t outputs = (int64_t)p.m * p.n;
+    if (p.k < 64 && p.m <= 32 && p.n <= 32 && (batch == 1 || outputs <= 256)) return true;
+    if (batch == 1 && p.m <= 128 && p.n <= 128 && p.n % 4 == 0 && p.k > 64 && p.k < 352 && p.k % 32) return true;
+    return p.k == 16 && outputs * batch >= (int64_t)1 << 20;
+}
 // Tile order of the grouped weight gradients: bands of 8 tile rows walked column by column when the group runs
 // unsplit (the workgroups one XCD runs together then share operand panels), row-major when it splits K.
 int group_band(int splits) { return splits == 1 ? 8 : 0; }
 }  // namespace
 
-// Thin products (one side at most 32: a classifier head's weight gradient, 9 x 768 over K = 4096 tokens) take the
-// 128 x 32 / 32 x 128 tiles. Products with fewer tiles than CUs (the classifier heads, small batches) split K into
-// slices of at least 32 k, up to about one workgroup per CU: their time is the chain of chunk loads each workgroup
-// waits for, not arithmetic.
+// Tiles of the guarded kernel: 128 x 32 / 32 x 128 where one side is at most 32, so that a thin product is not mostly padding.
+// Products with fewer tiles than CUs split K into slices of at least 32 k, up to about one workgroup per CU: their time is the
+// chain of chunk loads each workgroup waits for, not arithmetic.
 Choice choose(int m, int n, int k, int batch, int cus) {
     Choice c{64, 64, 1, k, 16};
     if (n <= 32) c = Choice{128, 32, 1, k, 16};
@@ -303,8 +318,8 @@ Choice choose(int m, int n, int k, int batch, int cus) {
 
 // Short sums over few tiles on the tile-exact fp32 kernels: whole 64 x 64 tiles, or 64 x 96 where those would be more than the
 // CUs, at most one per CU. A chunk of 32 k costs them 0.55 and 0.75 us, the split-operand kernel less but a longer start, so
-// the line lies at 288 (both operands K-contiguous, whose chunks go straight into LDS: 320), and lower where that kernel has
-// CUs left for k groups and splits, or whole rounds of four k groups (k = 256). Against it (us, k 160 / 224 / 288 / 320 / 384,
+// the line lies at 320 (64 x 64 tiles of operands that are not both K-contiguous, whose chunks do not go straight into LDS: 288),
+// and lower where that kernel has CUs left for k groups and splits, or whole rounds of four k groups (k = 256). Against it (us, k 160 / 224 / 288 / 320 / 384,
 // operands K-contiguous): 4096 x 384 8.7 / 9.6 / 11.2 / 12.2 / 13.7 here and 9.1 / 10.8 / 12.6 / 12.9 / 13.1 there, 1024 x 256 6.1
 // / 7.2 / 8.3 / 8.9 / 10.0 and 8.2 / 8.4 / 10.0 / 9.8 / 10.7, 64 x 64 5.7 / 6.8 / 7.9 / 8.5 / 9.5 and 7.9 / 8.0 / 8.2 / 7.8 /
 // 8.0; weight gradients of 1024 x 256 at k 256 / 288 / 320 8.7 / 9.3 / 10.0 and 8.3 / 10.7 / 10.1. With more than a tile per CU
@@ -320,7 +335,7 @@ static int short_tile(const Params &p, bool ta, bool tb, int batch, int cus) {
     for (const int bn : {64, 96}) {
         const int64_t tiles = (int64_t)(p.m / 64) * (p.n / bn) * batch;
         if (p.n % bn || tiles > cus) continue;
-        const int most = bn == 96 && tiles * 2 <= cus ? 160 : !tb || tiles * 8 < cus ? 288 : 320;
+        const int most = bn == 96 ? (tiles * 2 <= cus ? 160 : 320) : !tb || tiles * 8 < cus ? 288 : 320;
         return p.k <= most && (tb || p.k != 256) ? bn : 0;
     }
     return 0;
@@ -389,7 +404,7 @@ om_status launch_dense(om_ctx *ctx, Params p, bool ta, bool tb, int batch, const
         else launch_short<64>(p, ta, tb, batch, st);
         return OM_LAUNCH_CHECK(ctx, what);
     }
-    if (s_takes(p, ta, tb)) {
+    if (s_takes(p, ta, tb) && !general_wins(p, batch)) {
         const bool mask = p.mask != nullptr;
         const SChoice c = choose_s(1, &p.m, &p.n, p.k, batch, ctx->num_cus, !mask);
         p.splits = c.splits;

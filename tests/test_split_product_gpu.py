@@ -159,3 +159,17 @@ def test_short_sums_on_both_sides_of_the_rule(dev, ta, tb, m, n, k):
     want = A64 @ B64 + bias + c0
     bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + 2.0 ** -22 * (np.abs(bias) + np.abs(c0) + np.abs(want))
     assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", [(16, 16, 16), (32, 32, 63), (33, 32, 40), (128, 128, 65), (128, 100, 351), (129, 100, 163), (128, 128, 353),
+                                   (1024, 1024, 16), (1024, 1024, 17)])
+def test_small_products_on_both_sides_of_the_rule(dev, ta, tb, m, n, k):
+    """Products around the sizes up to which the guarded fp32 kernel runs, with bias and accumulation."""
+    rng = np.random.default_rng(m + k)
+    A, B, A64, B64 = operands(rng, ta, tb, m, n, k)
+    bias, c0 = rng.standard_normal(n).astype(np.float32), rng.standard_normal((m, n)).astype(np.float32)
+    got = product(dev, ta, tb, A, B, m, n, k, c0=c0.copy(), bias=bias, acc=1)
+    want = A64 @ B64 + bias + c0
+    bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + 2.0 ** -22 * (np.abs(bias) + np.abs(c0) + np.abs(want))
+    assert np.all(np.abs(got - want) <= bound)
