@@ -661,16 +661,61 @@ om_status sum_splits(om_ctx *ctx, const float *ws, int nsplit, int N, int H, int
     return OM_LAUNCH_CHECK(ctx, "conv2d split sum");
 }
 
+// The fp32 kernel's launch: 128 pixels x BM output channels a workgroup, chunks of 8 input channels, `nsplit` runs of them.
+struct Fp32Plan {
+    int R, ps, ns, BM, ntile, nsplit, cps;
+    int64_t tiles;
+};
+bool fp32_plan(const om_ctx *ctx, int N, int Cin, int H, int W, int Cout, Fp32Plan &f) {
+    const int P = H * W;
+    if (Cin % kFwdCk || Cout % 32 || W % 4 || (int64_t)N * Cin * P > INT32_MAX || (int64_t)N * Cout * P > INT32_MAX ||
+        (int64_t)Cout * 9 * Cin > INT32_MAX)
+        return false;
+    stage_geometry(W, kFwdPx, f.R, f.ps);
+    f.ns = stage_ns(kFwdCk, W, f.R);
+    if (!f.ns) return false;
+    f.BM = Cout % 64 == 0 ? 64 : 32;
+    f.ntile = (P + kFwdPx - 1) / kFwdPx;
+    f.tiles = (int64_t)f.ntile * (Cout / f.BM) * N;
+    // Fewer tiles than two per CU (small images): split the input channels, at least two chunks per split.
+    const int chunks = Cin / kFwdCk;
+    f.nsplit = 1, f.cps = chunks;
+    if (f.tiles < 2 * ctx->num_cus && chunks >= 4) {
+        int want = (int)((2 * ctx->num_cus + f.tiles - 1) / f.tiles);
+        if (want > chunks / 2) want = chunks / 2;
+        f.cps = (chunks + want - 1) / want;
+        f.nsplit = (chunks + f.cps - 1) / f.cps;
+    }
+    return true;
+}
+
+// Estimated us of either kernel, fitted to 740 shapes (1-48 images, 16-256 channels, widths 4-320; 80 % within 9 and 7 %): a
+// chunk's cost by the units staged for it and the multiplications, for the workgroups that share a CU, a start per round, and
+// the second pass over split sums.
+double split_time(const om_ctx *ctx, int64_t grid, int CB, int NW, int units, int lds, int nsplit, int cps, double outputs) {
+    const int64_t cus = ctx->num_cus, held = cus * ((160 << 10) / lds), share = (grid + cus - 1) / cus,
+                  rounds = (grid + held - 1) / held;
+    const double nw = NW / 8.0, first = 0.65 + nw * (0.58 * units + (CB == 2 ? 2.65 : 0.0)),
+                 more = nw * (0.76 * units + (CB == 2 ? 2.8 : 2.2));
+    return 1.5 + cps * (first * (double)rounds + more * (double)(share - rounds)) + 4.4 * (double)rounds +
+           (nsplit > 1 ? 1.6 + 2.8e-6 * outputs * nsplit : 0.0);
+}
+double fp32_time(const om_ctx *ctx, const Fp32Plan &f, double outputs) {
+    const double share = (double)((f.tiles * f.nsplit + ctx->num_cus - 1) / ctx->num_cus);
+    return 6.0 + f.cps * (0.05 + 0.06 * f.ns + share * (0.08 * f.ns + (f.BM == 64 ? 2.17 : 0.78))) + 1.65 * share +
+           (f.nsplit > 1 ? 1.9e-6 * outputs * f.nsplit : 0.0);
+}
+
 // The split-operand kernel (om_conv3_s.hpp): input channels in sixteens, output channels in thirty-twos, any width whose
 // staged rows fit the LDS. Blocks of 64 output channels halve the input's staging; those of 32 need half the weights' LDS,
 // for rows too wide otherwise. Eight wavefronts (256 pixels) or four, and runs of input channels whose partial sums a
 // second pass adds, as the fp32 kernel's are: the least rounds of workgroups over the CUs times chunks, a chunk of eight
 // wavefronts costing 4 (measured 7.5 us), of four 3, and the second pass 4. Measured against the fp32 kernel (us): 32 x 64
 // x 28 x 28 37.7 -> 27.4, 64 x 256 -> 512 channels at 8 x 8 160 -> 95, 2 x 64 at 112 x 112 34.8 -> 27.1, 1 x 64 at 28 x 28
-// 12.4 -> 10.2, 2 x 32 -> 64 at 32 x 280 35.5 -> 22.6. With one or two chunks of wide rows on a quarter of the CUs the
-// first chunk's loads are not hidden and the fp32 kernel's smaller tiles keep the lead (1 x 32 at 32 x 224: 11.4 against
-// 16.2 us; past 256 columns the latter's staging falls apart, 39 against 17 us): those stay there. The dearest shape that
-// does not: 16 x 128 -> 32 channels at 32 x 192, 384 workgroups on 256 CUs, 77 -> 84 us.
+// 12.4 -> 10.2, 2 x 32 -> 64 at 32 x 280 35.5 -> 22.6. Where the fp32 kernel's estimate is the lower one the call is left to
+// it: rows of 128 columns and more, whose staging is long, on part of the chip or in one round and a half (1 x 64 -> 32 at 32 x 224
+// 13.3 there and 15.7 here, 16 x 128 -> 32 at 32 x 192 80 and 86). Over the 740 shapes the choice is 0.2 % above the faster of the
+// two on average, and 10 % above the fp32 kernel at worst.
 bool split_conv(om_ctx *ctx, const float *x, const float *w, const float *bias, float *y, int N, int Cin, int H, int W,
                 int Cout, int acc, om_status *st, bool flip, bool relu, const Conv3Pool *pool, bool *pooled) {
     const int P = H * W;
@@ -697,8 +742,13 @@ bool split_conv(om_ctx *ctx, const float *x, const float *w, const float *bias, 
                 a.R = R, a.ntile = nt, a.nsplit = n, a.cps = cps;
             }
         }
-    if (!NW || (chunks <= 2 && units > 6 && W % 4 == 0 && W <= 256 && grid_n * 4 <= ctx->num_cus)) return false;
+    if (!NW) return false;
     const int NU = units <= 4 ? 4 : units <= 6 ? 6 : units <= 8 ? 8 : 12, lds = oc3::lds_bytes(a.R, W, CB);
+    const double outputs = (double)N * Cout * P;
+    Fp32Plan f;
+    if (fp32_plan(ctx, N, Cin, H, W, Cout, f) &&
+        fp32_time(ctx, f, outputs) < split_time(ctx, grid_n, CB, NW, units, lds, a.nsplit, a.cps, outputs))
+        return false;
     if (a.nsplit > 1) {
         *st = om::scratch2(ctx, sizeof(float) * (uint64_t)a.nsplit * N * Cout * P, &a.ws);
         if (*st) return true;
@@ -808,45 +858,28 @@ bool om_conv3_fwd(om_ctx *ctx, const float *x, const float *w, const float *bias
         return true;
     }
     if (split_conv(ctx, x, w, bias, y, N, Cin, H, W, Cout, acc, st, flip_weights, relu, pool, pooled)) return true;
-    if (Cin % kFwdCk || Cout % 32 || W % 4 || (int64_t)N * Cin * P > INT32_MAX || (int64_t)N * Cout * P > INT32_MAX ||
-        (int64_t)Cout * 9 * Cin > INT32_MAX)
-        return false;
-    int R, ps;
-    stage_geometry(W, kFwdPx, R, ps);
-    const int ns = stage_ns(kFwdCk, W, R);
-    if (!ns) return false;
-    const int BM = Cout % 64 == 0 ? 64 : 32;
+    Fp32Plan f;
+    if (!fp32_plan(ctx, N, Cin, H, W, Cout, f)) return false;
     // forward: the layer's W [Cout][Cin][9]; dX (flip): the layer's W [Cout_l][Cin_l][9], where this call's Cin is
     // Cout_l and its Cout is Cin_l (the kernel reads it flipped and transposed)
-    const int ntile = (P + kFwdPx - 1) / kFwdPx;
+    const int BM = f.BM, ns = f.ns, nsplit = f.nsplit;
     const size_t lds = sizeof(float) * (9 * (size_t)(BM == 64 ? w_tap_stride<64>() : w_tap_stride<32>()) +
-                                        (size_t)kFwdCk * ps);
-    const int64_t tiles = (int64_t)ntile * (Cout / BM) * N;
-    // Fewer tiles than two per CU (small images): split the input channels, at least two chunks per split.
-    const int chunks = Cin / kFwdCk;
-    int nsplit = 1, cps = chunks;
-    if (tiles < 2 * ctx->num_cus && chunks >= 4) {
-        int want = (int)((2 * ctx->num_cus + tiles - 1) / tiles);
-        if (want > chunks / 2) want = chunks / 2;
-        cps = (chunks + want - 1) / want;
-        nsplit = (chunks + cps - 1) / cps;
-    }
+                                        (size_t)kFwdCk * f.ps);
     float *ws = nullptr;
-    const int64_t total = (int64_t)N * Cout * P;
     if (nsplit > 1) {
-        *st = om::scratch2(ctx, sizeof(float) * (uint64_t)nsplit * total, &ws);
+        *st = om::scratch2(ctx, sizeof(float) * (uint64_t)nsplit * N * Cout * P, &ws);
         if (*st) return true;
     }
-    const dim3 grid((unsigned)(tiles * nsplit));
+    const dim3 grid((unsigned)(f.tiles * nsplit));
     const int rl = relu && nsplit == 1 ? 1 : 0;  // with splits the sum applies it
 #define OMC3(BM_, NS_)                                                                                             \
     if (BM == BM_ && ns == NS_) {                                                                                  \
         if (flip_weights)                                                                                          \
             hipLaunchKernelGGL((k_conv3_fwd<BM_, NS_, true>), grid, dim3(kThreads), lds, ctx->stream, x, w, bias, y, \
-                               Cin, Cout, H, W, R, ps, ntile, acc, N, nsplit, cps, ws, rl);                         \
+                               Cin, Cout, H, W, f.R, f.ps, f.ntile, acc, N, nsplit, f.cps, ws, rl);                 \
         else                                                                                                       \
             hipLaunchKernelGGL((k_conv3_fwd<BM_, NS_, false>), grid, dim3(kThreads), lds, ctx->stream, x, w, bias, \
-                               y, Cin, Cout, H, W, R, ps, ntile, acc, N, nsplit, cps, ws, rl);                      \
+                               y, Cin, Cout, H, W, f.R, f.ps, f.ntile, acc, N, nsplit, f.cps, ws, rl);              \
     }
     OMC3(64, 1) OMC3(64, 2) OMC3(64, 3) OMC3(64, 4) OMC3(64, 6) OMC3(64, 8)
     OMC3(32, 1) OMC3(32, 2) OMC3(32, 3) OMC3(32, 4) OMC3(32, 6) OMC3(32, 8)

@@ -1,6 +1,6 @@
 """The split-operand 3x3 convolution (csrc/om_conv3_s.hpp) at the sizes and values where it can go wrong: widths that are
-no multiple of 4, partial pixel tiles, both channel blocks, one chunk of channels and split channels, accumulation, and
-operands the three-way bf16 split does not carry, against float64 over the zero-padded input.
+no multiple of 4, wide rows (some of which the fp32 kernel takes), partial pixel tiles, both channel blocks, one chunk of channels and
+split channels, accumulation, and operands the three-way bf16 split does not carry, against float64 over the zero-padded input.
 
 Tolerance: the sequential-accumulation bound k 2^-24 sum |w||x| over the k = 9 Cin terms (the kernel's own rounding count
 is lower: one per 16 terms and six per 16 on sums 2^-8 as large), and a rounding of each later addition.
@@ -39,7 +39,7 @@ def turned(w):
 # (images, Cin, Cout, H, W): dX exchanges the channels
 SHAPES = [(1, 32, 32, 1, 1), (1, 32, 64, 3, 5), (2, 64, 32, 7, 7), (3, 96, 64, 5, 33), (1, 512, 64, 2, 3), (2, 32, 96, 19, 27),
           (40, 64, 64, 15, 17), (9, 32, 160, 31, 33), (300, 32, 32, 3, 3), (2, 32, 64, 4, 185), (1, 64, 32, 3, 189),
-          (1, 32, 64, 90, 62)]
+          (1, 32, 64, 90, 62), (1, 32, 64, 13, 224), (1, 64, 32, 8, 224), (2, 96, 32, 9, 256), (5, 32, 96, 12, 128), (2, 48, 64, 8, 192)]
 
 
 @pytest.mark.parametrize("N,Cin,Cout,H,W", SHAPES)
