@@ -117,3 +117,15 @@ class Dev:
 
 def ptr(t):
     return C.c_void_p(t.data_ptr()) if t is not None else None
+
+
+# Largest relative error of a product of two fp32 values by the six-term split (csrc/om_split.hpp): the dropped ml, lm and ll
+# are below 2^-24 (1 + 2^-9) of it, the sum of its halves rounds to 2^-24, and the five roundings of the small terms, 2^-7 as
+# large, add 2^-28.
+SPLIT_PRODUCT = 2.0 ** -23 * (1 + 2.0 ** -4)
+
+
+def full_significands(rng, shape):
+    """fp32 values that use all 24 bits of the significand, over 2^-8 .. 2^8."""
+    m = rng.integers(1 << 23, 1 << 24, shape).astype(np.float64) * rng.choice([-1.0, 1.0], shape)
+    return np.ldexp(m, rng.integers(-31, -15, shape)).astype(np.float32)

@@ -3,8 +3,9 @@ wrong: one pixel, odd numbers of eight-column groups, widths that are no multipl
 last row, slots with one and many items, several channel blocks, accumulation, and operands the three-way bf16 split does not
 carry, against float64 over the zero-padded input.
 
-Tolerance: the sequential-accumulation bound k 2^-24 sum |g||x| over the k = N H W terms, and a rounding of the later
-addition; the bias gradient is summed in double and rounded once.
+Tolerance: for edges and values the sequential-accumulation bound k 2^-24 sum |g||x| over the k = N H W terms, and a rounding of
+the later addition; for the precision itself, single products within 2^-23. The bias gradient is summed in double and rounded
+once.
 """
 import numpy as np
 import pytest
@@ -51,6 +52,23 @@ def test_edges(dev, N, Cin, Cout, H, W):
         assert np.all(np.abs(dev.get(DW) - ref) <= bound)
         if not acc:
             assert np.all(np.abs(dev.get(DB) - dbw) <= 2.0 ** -23 * np.abs(dbw) + 1e-12)
+
+
+@pytest.mark.parametrize("N,Cin,Cout,H,W", [(4100, 32, 64, 1, 1), (90, 64, 64, 7, 7), (26, 96, 64, 5, 33), (9, 32, 192, 19, 27), (40, 64, 64, 15, 17),
+                                            (6, 32, 64, 4, 185), (4, 32, 64, 16, 112), (450, 32, 64, 3, 3), (7, 32, 64, 9, 73)])
+def test_single_products(dev, N, Cin, Cout, H, W):
+    """One pixel of g in each output channel, at the borders, at the edges of column groups and segments and inside, so every result is
+    one product of two full significands (or the zero beside the image) and shows each of the six terms: a lost or misplaced plane
+    leaves 2^-17 or more (test_split_terms.py)."""
+    rng = np.random.default_rng(N + W)
+    x, g, i = gpu_util.full_significands(rng, (N, Cin, H, W)), np.zeros((N, Cout, H, W), np.float32), np.arange(Cout)
+    cols = np.array([0, W - 1, 7, 8, 9, 15, 23, 24, 31, 32, 33, W // 2, W - 2]) % W
+    g[i * 5 % N, i, i * 3 % H, cols[i % len(cols)]] = gpu_util.full_significands(rng, Cout)
+    DW = dev.empty((Cout, Cin, 3, 3))
+    dev.call("om_conv2d_bwd", dev.put(g), dev.put(x), dev.put(np.zeros(DW.shape, np.float32)), None, DW, None, N, Cin, H, W, Cout, 3, 3, 1,
+             1, 0, 0)
+    want = dw64(g, x)
+    assert np.all(np.abs(dev.get(DW) - want) <= gpu_util.SPLIT_PRODUCT * np.abs(want))
 
 
 def test_values_the_split_does_not_carry(dev):

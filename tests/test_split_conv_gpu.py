@@ -2,8 +2,9 @@
 no multiple of 4, wide rows (some of which the fp32 kernel takes), partial pixel tiles, both channel blocks, one chunk of channels and
 split channels, accumulation, and operands the three-way bf16 split does not carry, against float64 over the zero-padded input.
 
-Tolerance: the sequential-accumulation bound k 2^-24 sum |w||x| over the k = 9 Cin terms (the kernel's own rounding count
-is lower: one per 16 terms and six per 16 on sums 2^-8 as large), and a rounding of each later addition.
+Tolerance: for edges and values the sequential-accumulation bound k 2^-24 sum |w||x| over the k = 9 Cin terms (the kernel's own
+rounding count is lower: one per 16 terms and five per 16 on sums 2^-7 as large), and a rounding of each later addition; for the
+precision itself, single products within 2^-23.
 """
 import time
 
@@ -64,6 +65,28 @@ def test_edges(dev, N, Cin, Cout, H, W):
     want = conv64(g, turned(w)) + dx0
     bound = 9 * Cout * 2.0 ** -24 * conv64(np.abs(g), turned(np.abs(w))) + 2.0 ** -22 * (np.abs(want) + np.abs(dx0))
     assert np.all(np.abs(dev.get(DX) - want) <= bound)
+
+
+@pytest.mark.parametrize("N,Cin,Cout,H,W", [(64, 32, 32, 7, 7), (64, 64, 64, 5, 33), (96, 96, 160, 19, 27), (40, 64, 64, 15, 17),
+                                            (24, 32, 64, 4, 185), (32, 256, 64, 3, 5), (32, 64, 64, 56, 56)])
+def test_single_products(dev, N, Cin, Cout, H, W):
+    """One element in each image, at the borders and inside, so every result is one product of two full significands and shows each
+    of the six terms: a lost or misplaced plane leaves 2^-17 or more (test_split_terms.py)."""
+    rng = np.random.default_rng(N + W)
+    w = gpu_util.full_significands(rng, (Cout, Cin, 3, 3))
+
+    def images(chans):
+        x, i = np.zeros((N, chans, H, W), np.float32), np.arange(N)
+        rows, cols = np.array([0, H - 1, H // 2, 1 % H])[i % 4], np.array([0, W - 1, W // 2, 7 % W, 8 % W])[i % 5]
+        x[i, (i * 7) % chans, rows, cols] = gpu_util.full_significands(rng, N)
+        return x
+
+    x, g = images(Cin), images(Cout)
+    X, Wd, Y, DX = dev.put(x), dev.put(w), dev.empty(g.shape), dev.empty(x.shape)
+    dev.call("om_conv2d_fwd", X, Wd, None, Y, N, Cin, H, W, Cout, 3, 3, 1, 1)
+    dev.call("om_conv2d_bwd", dev.put(g), X, Wd, DX, dev.empty(w.shape), None, N, Cin, H, W, Cout, 3, 3, 1, 1, 0, 0)
+    for got, want in ((dev.get(Y), conv64(x, w)), (dev.get(DX), conv64(g, turned(w)))):
+        assert np.all(np.abs(got - want) <= gpu_util.SPLIT_PRODUCT * np.abs(want))
 
 
 @pytest.mark.parametrize("N,C,H,W", [(6, 32, 17, 19), (1, 64, 6, 9)])

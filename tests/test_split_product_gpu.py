@@ -1,10 +1,11 @@
 """The split-operand product (csrc/om_gemm_s.hpp) at the sizes and values where it can go wrong: partial tiles in both
 directions, K tails and uneven k groups, the last partial quad of columns, split K with its reduce, odd leading
-dimensions, and operands the three-way bf16 split does not carry (infinities, NaN, values past the largest bf16, values
-whose low part underflows), against float64.
+dimensions, operands the three-way bf16 split does not carry (infinities, NaN, values past the scaled range) and tiny ones,
+and the sizes on either side of the dispatch's rules, against float64.
 
-Tolerance: the sequential-accumulation bound k 2^-24 |A||B| that test_gemm_parity holds the product to (the kernel's own
-rounding count is lower: one per 16 terms and six per 16 on sums 2^-8 as large).
+Tolerance: for edges and values, where a wrong index shows, the sequential-accumulation bound k 2^-24 |A||B| that
+test_gemm_parity holds the product to (the kernel's own rounding count is lower: one per 16 terms and five per 16 on sums
+2^-7 as large); for the precision itself, single products within 2^-23 and the measured error of long sums.
 """
 import numpy as np
 import pytest
@@ -54,6 +55,27 @@ def test_edges(dev, ta, tb, m, n, k):
     assert np.all(np.abs(got[:, :n] - want) <= bound)
 
 
+# Every tile shape of the kernel, whole and ragged tiles, split K or not (on 256 CUs).
+TILES = [(6144, 1003, 64), (6144, 1024, 64), (3000, 1536, 64), (3072, 1536, 64), (3000, 1003, 64), (3072, 1024, 64), (2050, 1003, 64),
+         (1536, 1536, 64), (1500, 1003, 96), (1536, 1024, 96), (2050, 512, 96), (1000, 192, 768), (768, 1536, 384), (1536, 96, 768),
+         (64, 37, 96), (64, 37, 512), (256, 384, 384), (384, 192, 768), (64, 37, 64), (64, 37, 391), (1536, 1024, 64), (64, 64, 384)]
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("m,n,k", TILES)
+def test_single_products(dev, ta, tb, m, n, k):
+    """A has one element in each row, so every result is one product of two full significands and shows each of the six terms: a
+    lost or misplaced plane leaves 2^-17 or more (test_split_terms.py)."""
+    rng = np.random.default_rng(m + n + k)
+    at = (np.arange(m) * 29) % k
+    A64, a = np.zeros((m, k), np.float32), gpu_util.full_significands(rng, m)
+    A64[np.arange(m), at] = a
+    B = gpu_util.full_significands(rng, (n, k) if tb else (k, n))
+    got = product(dev, ta, tb, np.ascontiguousarray(A64.T) if ta else A64, B, m, n, k)
+    want = a.astype(np.float64)[:, None] * (B.T if tb else B)[at]
+    assert np.all(np.abs(got - want) <= gpu_util.SPLIT_PRODUCT * np.abs(want))
+
+
 @pytest.mark.parametrize("ta,tb", LAYOUTS)
 @pytest.mark.parametrize("m,n,k", [(130, 70, 200), (512, 384, 384)])
 def test_values_the_split_does_not_carry(dev, ta, tb, m, n, k):
@@ -68,7 +90,7 @@ def test_values_the_split_does_not_carry(dev, ta, tb, m, n, k):
     put(m - 1, k - 1, -np.inf)
     put(40, k // 2, np.nan)
     put(70, 9, 3.4e38)  # finite, past the largest bf16
-    # one row, and elsewhere one column, of values whose low parts underflow
+    # one row, and elsewhere one column, of tiny values
     for c in range(k):
         put(100, c, A64[100, c] * 1e-36)
     if tb:
@@ -173,3 +195,15 @@ def test_small_products_on_both_sides_of_the_rule(dev, ta, tb, m, n, k):
     want = A64 @ B64 + bias + c0
     bound = k * 2.0 ** -24 * (np.abs(A64) @ np.abs(B64)) + 2.0 ** -22 * (np.abs(bias) + np.abs(c0) + np.abs(want))
     assert np.all(np.abs(got - want) <= bound)
+
+
+@pytest.mark.parametrize("ta,tb", LAYOUTS)
+@pytest.mark.parametrize("k,most", [(384, 1.7e-7), (4096, 4.2e-7)])
+def test_sums_are_closer_than_the_fp32_instruction(dev, ta, tb, k, most):
+    """The 2-norm error of sums of normal products in one chain: one and a half times what was measured (1.1e-7, 2.7e-7), and below the
+    fp32 instruction's (3.5e-7, 1.1e-6), whose sums round once per product or four."""
+    m, n = 3072, 1536
+    A, B, A64, B64 = operands(np.random.default_rng(k), ta, tb, m, n, k)
+    got = product(dev, ta, tb, A, B, m, n, k)[::61].astype(np.float64)
+    want = A64[::61] @ B64
+    assert np.linalg.norm(got - want) <= most * np.linalg.norm(want)
