@@ -1,31 +1,31 @@
-// The dense product's kernel: fp32 operands multiplied on the bf16 matrix cores without losing a bit of them.
+// The dense product's kernel: fp32 operands multiplied on the bf16 matrix cores from three parts each that hold all of
+// their bits.
 //
-// What bounds it and why this form: v_mfma_f32_16x16x4_f32 tops out at 157 TFLOP/s, v_mfma_f32_16x16x32_bf16 at 16
-// times that. Every fp32 operand is split exactly into three bf16 values, x = h + m + l (8 + 8 + 8 significand bits,
-// each the rounding of what the previous ones leave), and the product keeps the six terms hh, hm, mh, hl, lh, mm; the
-// dropped ml, lm, ll are below 2^-25 of |x||y|, under half an ulp of the product. hh accumulates in one fp32
-// accumulator and the five small terms in another, so the large sum takes one rounding per 32 products instead of one
-// per product or four. Measured against 64-bit sums over K = 128 .. 16384 (normal, all-positive and wide-ranging
-// operands) the relative error is 0.32-0.43 of the fp32 instruction's (K 384: 1.07e-7 against 3.5e-7; K 16384: 8.1e-7
-// against 2.3e-6).
+// What bounds it and why this form: v_mfma_f32_16x16x4_f32 tops out at 157 TFLOP/s, v_mfma_f32_32x32x16_bf16 at 16 times
+// that. Every fp32 operand is split exactly into three bf16 values, x = h + m + l (8 + 8 + 8 significand bits, each the
+// rounding of what the previous ones leave), and the product keeps the six terms hh, hm, mh, hl, lh, mm; the dropped ml, lm
+// and ll are together below 2^-24 (1 + 2^-9) of |x||y| (2^-24.15 found), half an ulp of the product. hh accumulates in one
+// fp32 accumulator and the five small terms in another, so the large sum takes one rounding per 16 products instead of one
+// per product or four. Against 64-bit sums of normal operands the 2-norm error is 1.1e-7 at K = 384 and 2.7e-7 at 4096, the
+// fp32 instruction's 3.5e-7 and 1.1e-6.
 //
-// Operands are scaled by 2^24 on their way in, so no part of the smallest subnormal underflows, and the sums by 2^-48 on their
-// way out (om_split.hpp). What the scaled range does not hold takes the fp32 instruction: infinities, NaN, operands of 2^104
-// and sums of 2^80 leave a non-finite sum, and a wavefront that finds one among its finished sums recomputes its tile with
-// v_mfma_f32_32x32x2_f32 straight from global memory, so such values come out as that instruction gives them.
+// Operands are scaled by 2^24 on their way in, so no part of the smallest subnormal underflows, and the sums by 2^-48 on
+// their way out (om_split.hpp). What the scaled range does not hold takes the fp32 instruction: infinities, NaN, operands of
+// 2^104 and sums of 2^80 leave a non-finite sum, and a wavefront that finds some among its finished sums computes its tile
+// again with v_mfma_f32_32x32x2_f32 straight from global memory and takes those sums from there.
 //
-// A workgroup is MG x KG wavefronts and computes BM x BN = (16 TM MG) x (16 TN) of C. Each wavefront owns 16 TM rows
-// and all BN columns, so its A fragments are used by no other wavefront: it loads them from global memory straight
-// into the MFMA layout and splits them in registers. B is split once per workgroup on its way into LDS, in fragment
-// order (three bf16 planes; a wavefront's fragment read is 64 consecutive 16-byte slots), double-buffered with one
-// barrier per 32 k. KG > 1 wavefront groups take every KG-th 32-k step each and their sums are added through LDS in
-// group order: a product with few tiles then keeps four wavefronts per CU busy.
+// A workgroup is MG x KG wavefronts and computes BM x BN = (32 MG) x (32 TN) of C. Each wavefront owns 32 rows and all BN
+// columns, so its A fragments are used by no other wavefront: it loads them from global memory straight into the MFMA layout
+// and splits them in registers. B is split once per workgroup on its way into LDS, in fragment order (three bf16 planes; a
+// wavefront's fragment read is 64 consecutive 16-byte slots), double-buffered with one barrier per 32 k. KG > 1 wavefront
+// groups take every KG-th 32-k step each and their sums are added through LDS in group order: a product with few tiles then
+// keeps four wavefronts per CU busy.
 //
-// The MFMA's first operand is B and its second A, so lane l holds C at row l % 16 and the four columns
-// 4 (l / 16) .. + 3 of each 16 x 16 block: the epilogue reads and writes float4.
+// The MFMA's first operand is B and its second A, so lane l holds C at row l % 32 and columns 8 q + 4 (l / 32) .. + 3 (q =
+// 0 .. 3) of each 32 x 32 block.
 //
-// The k of a 32-step are permuted alike for both operands: lane group g (= l / 16) and element e hold
-// k = 16 (e / 4) + 4 g + (e % 4), so the 16-byte loads of a K-contiguous row cover 64 consecutive bytes.
+// The k of a 32-step are permuted alike for both operands: lane group g (= l / 32) and element e of 16 hold k = 8 (e / 4) +
+// 4 g + e % 4, so a lane's 16-byte loads of a K-contiguous row and its pair's cover 32 consecutive bytes.
 #pragma once
 
 #include "om_gemm_core.hpp"
@@ -35,9 +35,6 @@ namespace omg {
 namespace gs {
 
 using namespace oms;
-
-// k of element e (0 .. 15) in lane group g, relative to its 32-step; elements 8 h .. 8 h + 7 are MFMA h's.
-__device__ __forceinline__ int kof(int g, int e) { return 8 * (e >> 2) + 4 * g + (e & 3); }
 
 // ------------------------------------------------------------------------------------------------------------ loads
 // Byte offsets from a uniform pointer stay in 32 bits (the host checks them), so a load is one instruction.

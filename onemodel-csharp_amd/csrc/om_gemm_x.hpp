@@ -1,9 +1,8 @@
 // Tile-exact fp32 MFMA GEMM for gfx950, for products that fill at most one round of 64-row tiles with short sums
-// (launch_short in om_gemm.hip holds the rule and its measurements): their time is the chain of loads, where splitting
+// (short_tile in om_gemm.hip holds the rule and its measurements): their time is the chain of loads, where splitting
 // operands costs more than the faster matrix instruction gives.
 //
-// Preconditions, checked on the host: every tile is full (m % BM == 0, n % BN == 0), every split's K range is a
-// multiple of BKT, operands are 16-byte aligned with leading dimensions (and batch strides) multiples of 4. With
+// Preconditions, checked on the host: every tile is full (m % BM == 0, n % BN == 0), K is a multiple of BKT, operands are 16-byte aligned with leading dimensions (and batch strides) multiples of 4. With
 // those, the main loop carries no bounds logic at all: each thread issues a fixed list of float4 global loads and
 // LDS stores per chunk.
 //
@@ -16,7 +15,7 @@
 // Operand layouts in LDS: K layout [rows][BKT] with XOR-swizzled float4 chunks (kaddr), R layout [BKT][rows+4]. For an
 // R-layout operand the wavefront's 16-row (or 16-column) MFMA blocks are interleaved: block i of a wavefront's TX
 // blocks covers rows {TX*c + i}, so the TX fragments a lane needs for one k sit side by side and arrive in one wide
-// LDS read (b64 / b96 / b128) instead of TX separate ones; the epilogue maps rows and columns back accordingly, and
+// LDS read (b64 / b96) instead of TX separate ones; the epilogue maps rows and columns back accordingly, and
 // for an interleaved B a lane's TX output columns are adjacent, so C is written with wide stores.
 #pragma once
 
@@ -26,27 +25,24 @@ namespace omg {
 namespace gx {
 
 // K layout in LDS: row r keeps its BKT values with stride BKT (no pad), its float4 chunks permuted by an XOR with
-// kswz(r). A 16-lane phase of the b128 stores (two rows of 8 chunks at BKT 32, one row of 16 chunks at BKT 64) and
-// of the fragment reads (16 rows, one chunk each) then covers 16 distinct 4-bank groups of the 64 LDS banks; the
+// kswz(r). A 16-lane phase of the b128 stores (two rows of 8 chunks) and of the fragment reads (16 rows, one chunk
+// each) then covers 16 distinct 4-bank groups of the 64 LDS banks; the
 // padded layout [rows][BKT + 4] let the two rows of a store phase overlap on four banks.
 template <int BKT>
 __device__ __forceinline__ int kswz(int r) {
-    static_assert(BKT == 32 || BKT == 64, "K-layout swizzle is defined for 32- and 64-wide chunks");
-    return BKT == 32 ? ((r >> 1) & 7) : (r & 15);
+    static_assert(BKT == 32, "K-layout swizzle is defined for 32-wide chunks");
+    return (r >> 1) & 7;
 }
 template <int BKT>
 __device__ __forceinline__ int kaddr(int r, int chunk) {
     return r * BKT + 4 * (chunk ^ kswz<BKT>(r));
 }
 
-// Exact loader of one operand chunk: ROWS x BKT values (KCONTIG: rows contiguous along k; else along the rows),
-// spread over NTH threads (a chunk that does not split evenly leaves whole wavefronts idle on the last load).
-template <int ROWS, int BKT, bool KCONTIG, int NTH = NT>
+// Exact loader of one operand chunk: ROWS x BKT values (KCONTIG: rows contiguous along k; else along the rows).
+template <int ROWS, int BKT, bool KCONTIG>
 struct Ld {
-    static constexpr int TOT = ROWS * BKT / 4;
-    static_assert(TOT % 64 == 0, "a chunk must split into whole wavefronts");
-    static constexpr int NV = (TOT + NTH - 1) / NTH;
-    static constexpr bool RAGGED = TOT % NTH != 0;
+    static constexpr int NV = ROWS * BKT / 4 / NT;
+    static_assert(ROWS * BKT % (4 * NT) == 0, "a chunk splits evenly over the threads");
     static constexpr int LDSZ = KCONTIG ? ROWS * BKT : BKT * (ROWS + PAD);
     const float *base;  // operand origin of this tile (row r0, k 0)
     int64_t ld;
@@ -56,8 +52,7 @@ struct Ld {
     __device__ __forceinline__ Ld(const float *b, int64_t ld_, int r0) : ld(ld_) {
 #pragma unroll
         for (int i = 0; i < NV; i++) {
-            int f = threadIdx.x + i * NTH;
-            if (RAGGED && f >= TOT) f = TOT - 1;  // unused: the load and store below are skipped for it
+            const int f = threadIdx.x + i * NT;
             if constexpr (KCONTIG) {
                 int r = f / (BKT / 4), kq = (f % (BKT / 4)) * 4;
                 goff[i] = (int)(r * ld) + kq;
@@ -73,15 +68,11 @@ struct Ld {
     __device__ __forceinline__ void fetch(floatx4 (&v)[NV], int k0) const {
         const float *p = base + (KCONTIG ? (int64_t)k0 : (int64_t)k0 * ld);
 #pragma unroll
-        for (int i = 0; i < NV; i++)
-            if (!RAGGED || i + 1 < NV || (int)threadIdx.x + i * NTH < TOT)
-                v[i] = *reinterpret_cast<const floatx4 *>(p + goff[i]);
+        for (int i = 0; i < NV; i++) v[i] = *reinterpret_cast<const floatx4 *>(p + goff[i]);
     }
     __device__ __forceinline__ void put(const floatx4 (&v)[NV], float *T) const {
 #pragma unroll
-        for (int i = 0; i < NV; i++)
-            if (!RAGGED || i + 1 < NV || (int)threadIdx.x + i * NTH < TOT)
-                *reinterpret_cast<floatx4 *>(T + soff[i]) = v[i];
+        for (int i = 0; i < NV; i++) *reinterpret_cast<floatx4 *>(T + soff[i]) = v[i];
     }
 };
 
@@ -100,16 +91,7 @@ __device__ __forceinline__ void read_frag(float (&f)[4][TX], const float *T, int
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             const float *p = &T[(blk * 16 + kl * 4 + s) * (ROWS + PAD) + w0 + TX * l16];
-            if constexpr (TX % 4 == 0) {
-#pragma unroll
-                for (int x = 0; x < TX; x += 4) {
-                    floatx4 v = *reinterpret_cast<const floatx4 *>(p + x);
-                    f[s][x] = v[0];
-                    f[s][x + 1] = v[1];
-                    f[s][x + 2] = v[2];
-                    f[s][x + 3] = v[3];
-                }
-            } else if constexpr (TX % 2 == 0) {
+            if constexpr (TX % 2 == 0) {
 #pragma unroll
                 for (int x = 0; x < TX; x += 2) {
                     float2 v = *reinterpret_cast<const float2 *>(p + x);
@@ -125,12 +107,12 @@ __device__ __forceinline__ void read_frag(float (&f)[4][TX], const float *T, int
 }
 
 // Fused bias gradient of a weight-gradient product: column sums of A (transposed, staged [BKT][BM+4] in LDS) over
-// the k rows of each chunk, in double. Thread x of NTH sums column x % BM over rows x / BM, x / BM + NTH / BM, ...;
-// colsum_finish combines the NTH / BM row groups in order and writes the tile's BM sums.
-template <int BM, int BKT, int NTH>
+// the k rows of each chunk, in double. Thread x sums column x % BM over rows x / BM, x / BM + NT / BM, ...; finish
+// combines the NT / BM row groups in order and writes the tile's BM sums.
+template <int BM, int BKT>
 struct ColSum {
-    static constexpr int RG = NTH / BM;
-    static_assert(NTH % BM == 0 && BKT % RG == 0, "column sums need whole row groups");
+    static constexpr int RG = NT / BM;
+    static_assert(NT % BM == 0 && BKT % RG == 0, "column sums need whole row groups");
     double s = 0.0;
     __device__ __forceinline__ void add(const float *Ab) {
         const int c = threadIdx.x % BM, rg = threadIdx.x / BM;
@@ -138,7 +120,7 @@ struct ColSum {
         for (int kk = rg; kk < BKT; kk += RG) s += (double)Ab[kk * (BM + PAD) + c];
     }
     // Uses `sh` (RG * BM doubles of LDS, free when called) and ends with a barrier.
-    __device__ __forceinline__ void finish(const Params &p, double *sh, int m0, int split) {
+    __device__ __forceinline__ void finish(const Params &p, double *sh, int m0) {
         sh[threadIdx.x] = s;
         __syncthreads();
         if ((int)threadIdx.x < BM) {
@@ -146,12 +128,8 @@ struct ColSum {
 #pragma unroll
             for (int g = 1; g < RG; g++) t += sh[g * BM + threadIdx.x];
             const int row = m0 + threadIdx.x;
-            if (p.splits > 1) {
-                p.colsum_ws[(int64_t)split * p.m + row] = t;
-            } else {
-                float v = (float)t;
-                p.db[row] = p.db_acc ? p.db[row] + v : v;
-            }
+            float v = (float)t;
+            p.db[row] = p.db_acc ? p.db[row] + v : v;
         }
         __syncthreads();
     }
@@ -163,15 +141,13 @@ struct ColSum {
 // and the arithmetic follows in the reference's order: alpha, mask, bias, residual, GELU, then accumulate.
 template <int TM, int TN, bool AK, bool BKL, int GK>
 __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&acc)[TM][TN], float *C,
-                                              const float *mask, int m0, int n0, int wm0, int wn0, int l16, int kl,
-                                              int split) {
-    int colv[TN];
-#pragma unroll
-    for (int j = 0; j < TN; j++) colv[j] = n0 + wn0 + (BKL ? j * 16 + l16 : TN * l16 + j);
+                                              const float *mask, int m0, int n0, int wm0, int wn0, int l16, int kl) {
+    const int col0 = n0 + wn0 + (BKL ? l16 : TN * l16);
+    constexpr int CS = BKL ? 16 : 1;  // column step; constant, so that adjacent columns become one wide access
     float bcol[TN];
-    if (p.splits == 1 && p.bias && !p.bias_per_row) {
+    if (p.bias && !p.bias_per_row) {
 #pragma unroll
-        for (int j = 0; j < TN; j++) bcol[j] = p.bias[colv[j]];
+        for (int j = 0; j < TN; j++) bcol[j] = p.bias[col0 + CS * j];
     }
     double mse_acc = 0.0;
     // One MFMA row block (i) at a time keeps the gathered operands to 4 x TN registers each.
@@ -180,13 +156,6 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
         int rowv[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) rowv[r] = m0 + wm0 + (AK ? i * 16 + 4 * kl + r : TM * (4 * kl + r) + i);
-        if (p.splits > 1) {
-#pragma unroll
-            for (int r = 0; r < 4; r++)
-#pragma unroll
-                for (int j = 0; j < TN; j++) p.ws[((int64_t)split * p.m + rowv[r]) * p.n + colv[j]] = acc[i][j][r];
-            continue;
-        }
         float v[4][TN], t[4][TN];
 #pragma unroll
         for (int r = 0; r < 4; r++)
@@ -196,7 +165,7 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
 #pragma unroll
             for (int r = 0; r < 4; r++)
 #pragma unroll
-                for (int j = 0; j < TN; j++) t[r][j] = base[(int64_t)rowv[r] * ld + colv[j]];
+                for (int j = 0; j < TN; j++) t[r][j] = base[(int64_t)rowv[r] * ld + col0 + CS * j];
         };
         if (p.alpha != 1.0f) {
 #pragma unroll
@@ -237,7 +206,7 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
 #pragma unroll
                 for (int r = 0; r < 4; r++)
 #pragma unroll
-                    for (int j = 0; j < TN; j++) p.out2[(int64_t)rowv[r] * p.ld2 + colv[j]] = omd::gelu(v[r][j]);
+                    for (int j = 0; j < TN; j++) p.out2[(int64_t)rowv[r] * p.ld2 + col0 + CS * j] = omd::gelu(v[r][j]);
             } else if (p.epi == EPI_GELU_GRAD) {
                 gather(p.aux, p.ldaux);
 #pragma unroll
@@ -251,7 +220,7 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
                     for (int j = 0; j < TN; j++) {
                         float a, s;
                         omd::gelu_and_slope(v[r][j], a, s);
-                        p.out2[(int64_t)rowv[r] * p.ld2 + colv[j]] = s;
+                        p.out2[(int64_t)rowv[r] * p.ld2 + col0 + CS * j] = s;
                         v[r][j] = a;
                     }
             }
@@ -260,7 +229,7 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
 #pragma unroll
                 for (int r = 0; r < 4; r++)
 #pragma unroll
-                    for (int j = 0; j < TN; j++) p.out2[(int64_t)rowv[r] * p.ld2 + colv[j]] = omd::gelu_fast(v[r][j]);
+                    for (int j = 0; j < TN; j++) p.out2[(int64_t)rowv[r] * p.ld2 + col0 + CS * j] = omd::gelu_fast(v[r][j]);
             } else if (p.epi == EPI_GELU_GRAD_F) {
                 gather(p.aux, p.ldaux);
 #pragma unroll
@@ -274,7 +243,7 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
                     for (int j = 0; j < TN; j++) {
                         float a, s;
                         omd::gelu_and_slope_fast(v[r][j], a, s);
-                        p.out2[(int64_t)rowv[r] * p.ld2 + colv[j]] = s;
+                        p.out2[(int64_t)rowv[r] * p.ld2 + col0 + CS * j] = s;
                         v[r][j] = a;
                     }
             }
@@ -298,7 +267,7 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
 #pragma unroll
         for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int j = 0; j < TN; j++) C[(int64_t)rowv[r] * p.ldc + colv[j]] = v[r][j];
+            for (int j = 0; j < TN; j++) C[(int64_t)rowv[r] * p.ldc + col0 + CS * j] = v[r][j];
         if (p.mse_t) {  // d = stored value - target; the unit gradient 2 (d / n) as (d dsq) + (d dsq); sum of fl(d d)
             gather(p.mse_t, p.ldc);
 #pragma unroll
@@ -307,7 +276,7 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
                 for (int j = 0; j < TN; j++) {
                     const float d = v[r][j] - t[r][j];
                     const float u = p.mse_dsq * d;
-                    p.mse_unit[(int64_t)rowv[r] * p.ldc + colv[j]] = u + u;
+                    p.mse_unit[(int64_t)rowv[r] * p.ldc + col0 + CS * j] = u + u;
                     mse_acc += (double)(d * d);
                 }
         }
@@ -318,10 +287,9 @@ __device__ __forceinline__ void tile_epilogue(const Params &p, const floatx4 (&a
     }
 }
 
-// One tile (tm, tn) of batch-and-split index zz, by one workgroup of NT threads: the body of k_gemm_x and of the
-// grouped weight-gradient kernel.
+// One tile (tm, tn) of batch index z, by one workgroup of NT threads.
 template <int BM, int BN, int BKT, bool TA, bool TB, int GK>
-__device__ __forceinline__ void gemm_x_tile(const Params &p, int tm, int tn, int zz) {
+__device__ __forceinline__ void gemm_x_tile(const Params &p, int tm, int tn, int z) {
     constexpr bool AK = !TA, BKL = TB;  // operands in K layout
     constexpr int TM = BM / 32, TN = BN / 32, NB = BKT / 16;
     using LA = Ld<BM, BKT, AK>;
@@ -329,14 +297,12 @@ __device__ __forceinline__ void gemm_x_tile(const Params &p, int tm, int tn, int
     __shared__ __attribute__((aligned(16))) float As[2 * LA::LDSZ];
     __shared__ __attribute__((aligned(16))) float Bs[2 * LB::LDSZ];
 
-    if (zz >= p.batch * p.splits) return;
-    const int z = zz / p.splits, split = zz % p.splits;
+    if (z >= p.batch) return;
     const int outer = z / p.batch_div, inner = z % p.batch_div;
     const float *A = p.a + outer * p.sa_outer + inner * p.sa_inner;
     const float *B = p.b + outer * p.sb_outer + inner * p.sb_inner;
     const int m0 = tm * BM, n0 = tn * BN;
-    const int kbeg = split * p.k_split;
-    const int nk = (min(p.k, kbeg + p.k_split) - kbeg) / BKT;
+    const int nk = p.k / BKT;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, l16 = lane & 15, kl = lane >> 4;
     const int wm0 = (wv >> 1) * (BM / 2), wn0 = (wv & 1) * (BN / 2);
 
@@ -364,12 +330,11 @@ __device__ __forceinline__ void gemm_x_tile(const Params &p, int tm, int tn, int
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[s][i], fb[s][j], acc[i][j], 0, 0, 0);
     };
     // Bias gradient: the first column of tiles of a TN product sums its A chunks (A is [k][m] in LDS).
-    constexpr bool CS_OK = TA && (NT % BM == 0) && (BKT % (NT / BM) == 0);
-    ColSum<CS_OK ? BM : 64, BKT, NT> cs;
-    const bool do_cs = CS_OK && p.db && tn == 0;
+    ColSum<BM, BKT> cs;
+    const bool do_cs = TA && p.db && tn == 0;
     // Blocks 0 .. NB-2 of the chunk in (Ab, Bb): the fragments of block b+1 are read while block b multiplies.
     auto body = [&](const float *Ab, const float *Bb) {
-        if constexpr (CS_OK)
+        if constexpr (TA)
             if (do_cs) cs.add(Ab);
 #pragma unroll
         for (int blk = 0; blk + 1 < NB; blk++) {
@@ -385,12 +350,12 @@ __device__ __forceinline__ void gemm_x_tile(const Params &p, int tm, int tn, int
 
     if (nk > 0) {
         floatx4 ra0[LA::NV], rb0[LB::NV], ra1[LA::NV], rb1[LB::NV];
-        const int klast = kbeg + (nk - 1) * BKT;
+        const int klast = (nk - 1) * BKT;
         float *A0 = As, *A1 = As + LA::LDSZ, *B0 = Bs, *B1 = Bs + LB::LDSZ;
-        la.fetch(ra0, kbeg);
-        lb.fetch(rb0, kbeg);
-        la.fetch(ra1, min(kbeg + BKT, klast));
-        lb.fetch(rb1, min(kbeg + BKT, klast));
+        la.fetch(ra0, 0);
+        lb.fetch(rb0, 0);
+        la.fetch(ra1, min(BKT, klast));
+        lb.fetch(rb1, min(BKT, klast));
         la.put(ra0, A0);
         lb.put(rb0, B0);
         __syncthreads();
@@ -414,8 +379,8 @@ __device__ __forceinline__ void gemm_x_tile(const Params &p, int tm, int tn, int
         // Both halves of the loop body always run (loads past the last chunk are clamped to it), so the body has
         // no branch: a branchy body lets the compiler merge the halves and index the register sets dynamically.
         for (; t + 2 < nk; t += 2) {
-            OMG_X_HALF(ra0, rb0, ra1, rb1, A0, B0, A1, B1, kbeg + (t + 2) * BKT)
-            OMG_X_HALF(ra1, rb1, ra0, rb0, A1, B1, A0, B0, kbeg + (t + 3) * BKT)
+            OMG_X_HALF(ra0, rb0, ra1, rb1, A0, B0, A1, B1, (t + 2) * BKT)
+            OMG_X_HALF(ra1, rb1, ra0, rb0, A1, B1, A0, B0, (t + 3) * BKT)
         }
         const float *Al = A0, *Bl = B0;
         if (nk - t == 2) {
@@ -428,23 +393,23 @@ __device__ __forceinline__ void gemm_x_tile(const Params &p, int tm, int tn, int
         body(Al, Bl);
         mm(fa1, fb1);
     }
-    if constexpr (CS_OK)
-        if (p.db && tn == 0) {  // uniform over the workgroup
+    if constexpr (TA)
+        if (do_cs) {  // uniform over the workgroup
             __syncthreads();
-            cs.finish(p, reinterpret_cast<double *>(As), m0, split);
+            cs.finish(p, reinterpret_cast<double *>(As), m0);
         }
 
     float *C = p.c + outer * p.sc_outer + inner * p.sc_inner;
     const float *mask = p.mask ? p.mask + outer * p.mask_outer_stride : nullptr;
-    tile_epilogue<TM, TN, AK, BKL, GK>(p, acc, C, mask, m0, n0, wm0, wn0, l16, kl, split);
+    tile_epilogue<TM, TN, AK, BKL, GK>(p, acc, C, mask, m0, n0, wm0, wn0, l16, kl);
 }
 
 template <int BM, int BN, int BKT, bool TA, bool TB, int GK = 0>
 __global__ void __launch_bounds__(NT) k_gemm_x(Params p) {
     OM_LDS_POISON();
-    int tm, tn, zz;
-    tile_coords(p, p.n / BN, p.m / BM, tm, tn, zz);
-    gemm_x_tile<BM, BN, BKT, TA, TB, GK>(p, tm, tn, zz);
+    int tm, tn, z;
+    tile_coords(p, p.n / BN, p.m / BM, tm, tn, z);
+    gemm_x_tile<BM, BN, BKT, TA, TB, GK>(p, tm, tn, z);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
@@ -481,7 +446,7 @@ __device__ __forceinline__ void dma_chunk(const float *src, int64_t ld, unsigned
 }
 
 template <int BM, int BN, int BKT, int GK>
-__device__ __forceinline__ void gemm_xd_tile(const Params &p, int tm, int tn, int zz) {
+__device__ __forceinline__ void gemm_xd_tile(const Params &p, int tm, int tn, int z) {
     constexpr int TM = BM / 32, TN = BN / 32, NB = BKT / 16;
     constexpr int SA = BM * BKT, SB = BN * BKT, STAGE = SA + SB;
     constexpr int PER = (BM + BN) * (BKT / 4) / 64 / 4;  // loads per wavefront and chunk
@@ -489,14 +454,12 @@ __device__ __forceinline__ void gemm_xd_tile(const Params &p, int tm, int tn, in
     // 64 floats of pad ahead of the stages: no stage starts at LDS address 0
     __shared__ __attribute__((aligned(16))) float S[64 + 3 * STAGE];
 
-    if (zz >= p.batch * p.splits) return;
-    const int z = zz / p.splits, split = zz % p.splits;
+    if (z >= p.batch) return;
     const int outer = z / p.batch_div, inner = z % p.batch_div;
     const int m0 = tm * BM, n0 = tn * BN;
     const float *A = p.a + outer * p.sa_outer + inner * p.sa_inner + (int64_t)m0 * p.lda;
     const float *B = p.b + outer * p.sb_outer + inner * p.sb_inner + (int64_t)n0 * p.ldb;
-    const int kbeg = split * p.k_split;
-    const int nk = (min(p.k, kbeg + p.k_split) - kbeg) / BKT;
+    const int nk = p.k / BKT;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, l16 = lane & 15, kl = lane >> 4;
     const int wm0 = (wv >> 1) * (BM / 2), wn0 = (wv & 1) * (BN / 2);
 
@@ -511,8 +474,8 @@ __device__ __forceinline__ void gemm_xd_tile(const Params &p, int tm, int tn, in
     constexpr int CH = BKT / 4;
     static_assert((256 / CH) % 16 == 0, "the swizzle repeats every 16 rows");
     const int slot0 = wv * 64 + lane, r0 = slot0 / CH, c0 = (slot0 % CH) ^ kswz<BKT>(r0);
-    const float *srcA = A + (int64_t)r0 * p.lda + kbeg + 4 * c0;
-    const float *srcB = B + (int64_t)r0 * p.ldb + kbeg + 4 * c0;
+    const float *srcA = A + (int64_t)r0 * p.lda + 4 * c0;
+    const float *srcB = B + (int64_t)r0 * p.ldb + 4 * c0;
     const unsigned wave = __builtin_amdgcn_readfirstlane(wv);
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void *)(S + 64) + wave * 1024u;
     auto issue = [&](int t, int st) {
@@ -562,15 +525,15 @@ __device__ __forceinline__ void gemm_xd_tile(const Params &p, int tm, int tn, in
 
     float *C = p.c + outer * p.sc_outer + inner * p.sc_inner;
     const float *mask = p.mask ? p.mask + outer * p.mask_outer_stride : nullptr;
-    tile_epilogue<TM, TN, true, true, GK>(p, acc, C, mask, m0, n0, wm0, wn0, l16, kl, split);
+    tile_epilogue<TM, TN, true, true, GK>(p, acc, C, mask, m0, n0, wm0, wn0, l16, kl);
 }
 
 template <int BM, int BN, int BKT, int GK = 0>
 __global__ void __launch_bounds__(NT) k_gemm_xd(Params p) {
     OM_LDS_POISON();
-    int tm, tn, zz;
-    tile_coords(p, p.n / BN, p.m / BM, tm, tn, zz);
-    gemm_xd_tile<BM, BN, BKT, GK>(p, tm, tn, zz);
+    int tm, tn, z;
+    tile_coords(p, p.n / BN, p.m / BM, tm, tn, z);
+    gemm_xd_tile<BM, BN, BKT, GK>(p, tm, tn, z);
 }
 
 }  // namespace gx

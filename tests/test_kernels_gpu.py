@@ -58,7 +58,7 @@ def test_mfma_fragment_layout(dev):
                                    # inner dimensions shorter than one MFMA step or chunk (masked k loads)
                                    (70, 50, 1), (33, 129, 3), (600, 2, 7),
                                    # C5's products: the FFN pair and the 768-wide projections over 4096 tokens, and
-                                   # the weight-gradient shapes with K = 4096 (the tuned table's C5 rows)
+                                   # a weight-gradient shape with K = 4096
                                    (4096, 3072, 768), (4096, 768, 3072), (4096, 768, 768), (3072, 768, 4096)])
 def test_gemm_parity(dev, T, ta, tb, m, n, k):
     rng = np.random.default_rng(m * 1000 + n + k)
@@ -291,9 +291,8 @@ def _fused_epilogues(dev, T, rows, inf, outf, mode):
     dev.call("om_linear_bwd_dx_gelu", G, W, HI, DH, rows, inf, outf)
     assert scaled(dev.get(DH), dh_ref) <= TOL
     # GeluGradBin applied to the epilogue kernel's own product: om_linear_bwd_dx_slope with a unit slope yields that
-    # product exactly (x * 1 = x) from the tile every epilogue launch of this shape takes. A plain om_linear_bwd may
-    # take a tile that carries no epilogue (the eight-wavefront 128 x 128 one at 4096 x 3072 x 768), whose partial
-    # sums combine in another order, so it is held to the GEMM tolerance only.
+    # product exactly (x * 1 = x) from the tile every epilogue launch of this shape takes. A plain om_linear_bwd is held
+    # to the GEMM tolerance only.
     ONES = dev.put(np.ones((rows, inf), np.float32))
     dev.call("om_linear_bwd_dx_slope", G, W, ONES, DA, rows, inf, outf)
     da_dev = dev.get(DA)
