@@ -157,8 +157,9 @@ om_status om_graph_destroy(om_graph *g);
 /* ---------------------------------------------------------------------------------------------- GEMM */
 /* C[m,n] = op(A)[m,k] * op(B)[k,n] (+ bias[n]) in fp32, for `batch` independent products: on the bf16 matrix cores
  * from operands split exactly into three bf16 parts (closer to the exact sum than the fp32 matrix instruction, which
- * short sums and operands the split does not carry still take). Row-major operands
- * with leading dimensions lda/ldb/ldc; trans_a means A is stored [k,m], trans_b means B is stored [n,k].
+ * short sums, small products and what the split's range does not hold still take: infinities, NaN, operands from 2^104
+ * and sums from 2^80 on, each result by its own operands alone). Row-major operands with leading dimensions
+ * lda/ldb/ldc; trans_a means A is stored [k,m], trans_b means B is stored [n,k].
  * accumulate != 0 adds the product into C (C = C + AB, one rounding of the finished dot product), the leaf
  * accumulation of Engine.AccumulateLeaf (Engine.cs:292-328). Replaces Dense.Gemm / Kernels.Gemm.Run
  * (Dense.cs:12-49, Gemm.cs:48). Batch item z reads A at a + (z / batch_div) * sa_outer + (z % batch_div) * sa_inner
